@@ -209,9 +209,11 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
                          const int32_t* offsets, int E, int64_t P, int slots, const moe_qweight* w0,
                          const moe_qweight* w1, uint16_t* out, hipStream_t stream);
 // Grouped dense (bf16) matmul over expert buckets (gather_mm): out[row_out[pos]]
-// = x[row_in[pos]] . w[e]^T (+ linear_bias[e]) for the rows of each slot record.
-int grouped_mm(const uint16_t* x, const int32_t* row_in, const int32_t* row_out, const int32_t* active, int slots,
-               const uint16_t* w, const uint16_t* linear_bias, int N, int K, uint16_t* out, hipStream_t stream);
+// = x[row_in[pos]] . w[e]^T (+ linear_bias[e]) for the rows of the token-tile
+// table (P pairs over at most `slots` non-empty experts).
+int grouped_mm(const uint16_t* x, const int32_t* row_in, const int32_t* row_out, const int32_t* tiles, int slots,
+               int64_t P, const uint16_t* w, const uint16_t* linear_bias, int N, int K, uint16_t* out,
+               hipStream_t stream);
 // y[T] = bf16(x . dequant(w)^T) for a single quantized row w (experts 1, N 1)
 int qrow(const uint16_t* x, int64_t T, const moe_qweight* w, uint16_t* y, hipStream_t stream);
 int swiglu(const uint16_t* g, const uint16_t* u, int64_t n, uint16_t* h, hipStream_t stream);

@@ -205,6 +205,33 @@ def test_gather_mm(E, N, K, batch, M, use_lhs, biased):
     assert_close(hbf(got), O.gather_mm(x, w, lhs, rhs, M, b), what="gather_mm")
 
 
+@pytest.mark.parametrize("N,K,counts", [
+    # bucket remainders (mod 128 rows) at both ends of every token-tile class
+    (256, 512, [128, 129, 160, 161, 192, 193, 224, 225, 255, 0, 1]),
+    (1030, 2048, [1200, 1300, 1, 900, 0, 700, 950, 1100]),  # 256-column tiles, N neither a multiple of 8 nor of 256
+    (264, 32, [64, 33, 31, 90]),    # one K step
+    (140, 96, [1, 0, 2, 40, 1, 0, 0, 3]),  # 32-row tiles (few rows per expert), one expert with two of them
+])
+def test_gather_mm_tiles(N, K, counts):
+    """Every tile kernel of the dense gather_mm at its edges against fp32 torch on the bf16 inputs.  Bound:
+    half a bf16 ulp of the result (2^-8 relative) plus 8 sqrt(K) 2^-24 times the summed magnitudes (two
+    fp32 sums in different orders)."""
+    E, batch = len(counts), sum(counts)
+    rng = np.random.default_rng(N + K)
+    rhs = np.repeat(np.arange(E, dtype=np.uint32), counts)
+    rng.shuffle(rhs)
+    lhs = rng.integers(0, batch, batch).astype(np.uint32)
+    w = dbf(W.normal_bf16(E, 2, E * N * K, 0.05).reshape(E, N, K))
+    x = dbf(W.normal_bf16(E, 100, batch * K, 1.0).reshape(batch, K))
+    got = moe.gather_mm(x, w, di32(lhs), di32(rhs)).float()[:, 0]
+    for e in range(E):
+        rows = torch.from_numpy(np.flatnonzero(rhs == e)).to(DEV)
+        xe = x[di32(lhs).long()[rows]].float()
+        ref, mag = xe @ w[e].float().T, xe.abs() @ w[e].float().abs().T
+        bound = 2.0 ** -8 * ref.abs() + 8.0 * K ** 0.5 * 2.0 ** -24 * mag
+        assert ((got[rows] - ref).abs() <= bound).all(), f"expert {e}: {counts[e]} rows"
+
+
 @pytest.mark.parametrize("kind,batch", [("q4", 16), ("q4", 1000), ("q6", 40), ("dense", 16), ("dense", 1000)])
 def test_gather_out_of_range_experts(kind, batch):
     """rhs entries >= E (outside the contract; the checker rejects them): those output rows are zeros,
