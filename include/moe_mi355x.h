@@ -24,9 +24,8 @@
  *             ones examples/convert.cpp:10 emits and examples/test_qbits.cpp:45
  *             runs gather_qmm at; its --bits option takes the others); K a
  *             multiple of 128 at 3 and 5 bits; group_size 32, 64 or 128.
- *             Widths other than 4 and 8, and group size 32, run on the
- *             per-16-row kernel at every bucket size (the large-bucket GEMM
- *             is 4/8-bit with groups of 64 or 128).
+ *             2, 3 and 5 bits run on the per-16-row kernel at every bucket
+ *             size (the large-bucket GEMM takes 4, 6 and 8 bits).
  *
  * Host code above this ABI (the C++ SwitchLinear / SwitchGLU classes in
  * lemon-mlx-engine_amd/host/) keeps the reference's module interface; this

@@ -744,8 +744,9 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   }
   // when gate|up runs the large-bucket GEMM, the bf16 router projection (which
   // reads every row of x anyway) also writes the group sums of x that GEMM needs
-  const bool fuse_sums =
-      !qrouter && moe::router_tile32(T, d->hidden) && moe::use_prefill(P, slots, &d->gate, &d->up);
+  // (groups of whole 64-wide K steps; groups of 32 take the group-sum pass)
+  const bool fuse_sums = !qrouter && d->gate.group_size % 64 == 0 && moe::router_tile32(T, d->hidden) &&
+                         moe::use_prefill(P, slots, &d->gate, &d->up);
   const moe::RouterGroupSums sums{reinterpret_cast<uint16_t*>(p.gsum), d->gate.group_size,
                                   moe::prefill_gsum_stride(&d->gate) / 16};
   const bool pf_up = moe::use_prefill(P, slots, &d->gate, &d->up);

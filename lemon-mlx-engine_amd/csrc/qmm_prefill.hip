@@ -8,8 +8,8 @@
 //     P[m,n,g] = sum_{k in g} x[m][k] (q[n][k] + OFF)    (one MFMA chain per group)
 //     X[m,g]   = sum_{k in g} x[m][k]                    (group sums, fp32)
 //     b'       = b - OFF * s
-// 4-bit codes enter the MFMA as the bf16 value 128 + q (bit pattern 0x4300|q,
-// so OFF = 128); 8-bit codes as bf16(q) (exact below 256, OFF = 0).  Both are
+// 4- and 6-bit codes enter the MFMA as the bf16 value 128 + q (bit pattern
+// 0x4300|q, so OFF = 128); 8-bit codes as bf16(q) (exact below 256, OFF = 0).  Both are
 // exact, and x * (q + OFF) is exact in the fp32 accumulator.  Each group's
 // partial P is folded into the fp32 accumulator with one FMA per output
 // (acc += s * P).  (Rounding s*q + b to a bf16 operand instead would cost up
@@ -30,12 +30,12 @@
 // memory path retires about one line access per two clocks), so every
 // instruction reads whole or half lines:
 //   * activations: BM rows x 64 bf16 per K step, 8 lanes per 128-byte row,
-//     straight to LDS (no VGPR staging) into a ring of 3 (4-bit) / 2 (8-bit)
-//     steps, shared by the four waves (one LDS-only barrier per step);
+//     straight to LDS (no VGPR staging) into a ring of 3 (4, 6 bits) / 2 (8
+//     bits) steps, shared by the four waves (one LDS-only barrier per step);
 //   * codes: 64 bytes per weight row at a time (two K steps at 4 bits, one at
-//     8), 4 lanes per row, straight to LDS into two slots private to each
-//     wave, which expands its own rows to bf16 operands in registers (4-bit:
-//     one v_perm + one v_and_or per two codes);
+//     8), 4 lanes per row, or a 6-bit step's 48 bytes, 3 lanes per row,
+//     straight to LDS into two slots private to each wave, which expands its
+//     own rows to bf16 operands in registers;
 //   * scales: 8 groups (16 bytes) of a weight row per lane into registers, the
 //     other weight tile's row taken from the lane 32 apart (v_permlane32_swap).
 // LDS chunks are XOR-swizzled 16-byte units, so that the 16 lanes a 128-bit
@@ -44,7 +44,14 @@
 //
 // K order.  Within a 64-wide step, lane half h (= lane/32) of the A and B
 // operands of substep s carries K = 32h + 8s + [0, 8): a lane's B operands for
-// the whole step are one 16-byte (4-bit) or 32-byte (8-bit) run of codes.
+// the whole step are one 16-byte (4-bit), 24-byte (6-bit) or 32-byte (8-bit)
+// run of codes.  With groups of 32, two per step, substeps 0, 1 carry K 16h + 8s
+// of the first group and 2, 3 the same of the second, so each group is a chain
+// of two MFMAs with a fold of its own (twice the fold FMAs).
+//
+// Which calls: whole blocks at the Qwen3 shape, against the per-16-row kernel
+// (us): 6 bits T = 256 291 -> 201, T = 2048 1369 -> 413; groups of 32 at 4 bits
+// T = 256 291 -> 178, T = 2048 1501 -> 381, at 8 bits T = 2048 1727 -> 416.
 //
 // Scheduling.  Blocks are numbered so that consecutive virtual tiles land on
 // the same XCD (the hardware deals workgroups round-robin over 8 XCDs): the N
@@ -92,8 +99,11 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 256;
 constexpr int kBN = 256;           // weight rows per workgroup
-constexpr int kChunkRow = 64;      // code bytes per weight row in one code chunk
-constexpr int kChunkBytes = 4096;  // one wave's 64 rows of a chunk
+// code bytes per weight row in one code chunk: two K steps at 4 bits, one at 6 and 8
+template <int BITS>
+constexpr int kChunkRowOf = BITS == 6 ? 48 : 64;
+template <int BITS>
+constexpr int kChunkBytesOf = 64 * kChunkRowOf<BITS>;  // one wave's 64 rows of a chunk
 
 // g * (1 / (1 + e^-g)) (the checker's form) with the hardware exp and
 // reciprocal (v_exp_f32, v_rcp_f32: 1 ulp each; a correctly rounded
@@ -151,6 +161,42 @@ __device__ __forceinline__ bf16x8 expand_q4_pairs(uint32_t w, uint32_t k4300) {
   return __builtin_bit_cast(bf16x8, o);
 }
 
+// eight 6-bit codes = bits 6j .. 6j+5 of the 48 bits at byte 6S of the lane's
+// 24-byte run d -> bf16 operand [128 + code j].  Pair order: two byte permutes
+// gather codes 0..3 and 4..7 into the two halves of a dword (codes 0, 1 at bits
+// 0 and 6 of X01's halves, codes 2, 3 at bits 4 and 10 of X23's), then a shift
+// and an AND-OR per pair (j, j + 4): 9 instructions, the 4-bit codes' 7 plus
+// the permutes.  Natural order: the 12-bit field of codes 2j, 2j + 1 is split.
+template <bool PAIRS, int S>
+__device__ __forceinline__ bf16x8 expand_q6(const uint32_t (&d)[6], uint32_t k4300) {
+  const uint32_t w0 = d[S + (S >> 1)], w1 = d[S + (S >> 1) + 1];  // the two dwords that hold bytes 6S .. 6S+5
+  u32x4 o;
+  if constexpr (PAIRS) {
+    const uint32_t x01 = __builtin_amdgcn_perm(w1, w0, S & 1 ? 0x06050302u : 0x04030100u);
+    const uint32_t x23 = __builtin_amdgcn_perm(w1, w0, S & 1 ? 0x07060403u : 0x05040201u);
+    o[0] = and_or(x01, 0x003f003fu, k4300);
+    o[1] = and_or(x01 >> 6, 0x003f003fu, k4300);
+    o[2] = and_or(x23 >> 4, 0x003f003fu, k4300);
+    o[3] = and_or(x23 >> 10, 0x003f003fu, k4300);
+  } else {
+    uint32_t f[4];
+    if constexpr ((S & 1) == 0) {
+      f[0] = w0;
+      f[1] = w0 >> 12;
+      f[2] = __builtin_amdgcn_alignbit(w1, w0, 24);
+      f[3] = w1 >> 4;
+    } else {
+      f[0] = w0 >> 16;
+      f[1] = __builtin_amdgcn_alignbit(w1, w0, 28);
+      f[2] = w1 >> 8;
+      f[3] = w1 >> 20;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o[j] = and_or(f[j] << 10, 0x003f0000u, and_or(f[j], 0x0000003fu, k4300));
+  }
+  return __builtin_bit_cast(bf16x8, o);
+}
+
 // eight 8-bit codes (two words, code j in byte j) -> bf16 operand [code j],
 // natural order or (PAIRS) pair order
 template <bool PAIRS>
@@ -176,8 +222,8 @@ __device__ __forceinline__ bf16x8 expand_q8(uint32_t w0, uint32_t w1) {
 template <int BITS, bool GLU, int MT>
 constexpr int prefill_lds_bytes() {
   constexpr int BM = 32 * MT;
-  constexpr int kAStages = BITS == 4 ? 3 : 2;
-  constexpr int kMain = kAStages * BM * 128 + 4 * 2 * kChunkBytes + (kAStages == 3 ? 0 : BM * 128);
+  constexpr int kAStages = BITS == 8 ? 2 : 3;
+  constexpr int kMain = kAStages * BM * 128 + 4 * 2 * kChunkBytesOf<BITS> + (kAStages == 3 ? 0 : BM * 128);
   constexpr int kOut = BM * ((GLU ? 128 : kBN) + 8) * 2;
   return kMain > kOut ? kMain : kOut;
 }
@@ -188,12 +234,15 @@ constexpr int prefill_lds_bytes() {
 // activations other than SwiGLU; without it the SwiGLU epilogue alone is
 // compiled (the selector's other branches, inlined into every tile height's
 // unrolled epilogue, doubled the kernel's code and cost ~4 % of gate|up).
-template <int BITS, bool GLU, int MT, bool PAIRS, bool GACT = false>
+// G32: groups of 32, two per K step (another K order, below, and two folds).
+template <int BITS, bool GLU, int MT, bool PAIRS, bool GACT, bool G32>
 __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const int e, const int row0,
                                              const int rows, const int ntile) {
   constexpr int BM = 32 * MT;
-  constexpr int OFF = BITS == 4 ? 128 : 0;
-  constexpr int kAStages = BITS == 4 ? 3 : 2;  // activation ring (steps)
+  constexpr int OFF = BITS == 8 ? 0 : 128;
+  constexpr int kAStages = BITS == 8 ? 2 : 3;  // activation ring (steps)
+  constexpr int kChunkRow = kChunkRowOf<BITS>, kChunkBytes = kChunkBytesOf<BITS>;
+  constexpr int kBI = BITS == 6 ? 3 : 4;       // DMA instructions per code chunk
   constexpr int kLead = kAStages - 1;          // steps the loads run ahead
   constexpr int kABytes = BM * 128;            // activation tile per stage: BM rows x 64 bf16
   constexpr int kSPC = BITS == 4 ? 2 : 1;      // K steps per code chunk
@@ -214,7 +263,7 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
   const int h = lane >> 5, l32 = lane & 31;
   const int KS = a.K >> 6;
   const int NCH = KS / kSPC;  // code chunks along K
-  const int gdiv = a.gs >> 6;
+  const int gdiv = a.gs >> 6;  // K steps per group (G32: not used)
   const int G = a.K / a.gs;
   const uint32_t wrow_bytes = static_cast<uint32_t>(a.K) * BITS / 8;
 
@@ -266,6 +315,21 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
     return static_cast<uint32_t>(GLU ? (i & 1) * 16 : i * 16) * wrow_bytes;
   };
   uint8_t* bring = lds + kLdsA + wave * (kBSlots * kChunkBytes);
+  // 6-bit: the 64 rows' 48-byte runs are 192 16-byte units, three per row; lane
+  // -> unit 64 i + lane of instruction i, stored in order (row pitch 48 bytes:
+  // the lanes' 8-byte reads spread over all banks).  A unit's row decides its
+  // matrix, so each lane carries its own address
+  const uint8_t* csrc[3] = {nullptr, nullptr, nullptr};
+  if constexpr (BITS == 6) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const int u = 64 * i + lane, r = u / 3;
+      int mat;
+      const int wr = code_row(64 * wave + r, mat);
+      csrc[i] = reinterpret_cast<const uint8_t*>(mat ? a.w[1] : a.w[0]) +
+                (static_cast<int64_t>(e) * a.N + wr) * wrow_bytes + 16 * (u - 3 * r);
+    }
+  }
 
   auto issue_a = [&](int ks, int stage) {  // stage = ks % kAStages; steps past the end re-read the last step (in bounds)
     const uint32_t kc = static_cast<uint32_t>(min(ks, KS - 1));
@@ -276,9 +340,14 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
   auto issue_b = [&](int q) {
     const uint32_t qc = static_cast<uint32_t>(min(q, NCH - 1));
     uint8_t* dst = bring + (q % kBSlots) * kChunkBytes;
+    if constexpr (BITS == 6) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      buffer_load_lds16(wrs[GLU ? i >> 1 : 0], coff, qc * kChunkRow + crow_step(i), dst + i * 1024);
+      for (int i = 0; i < 3; ++i) load_lds16(csrc[i] + qc * kChunkRow, dst + i * 1024);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        buffer_load_lds16(wrs[GLU ? i >> 1 : 0], coff, qc * kChunkRow + crow_step(i), dst + i * 1024);
+    }
   };
 
   // ---- scales: lane (l32, h) holds 8 groups of weight row (nt = h, l32) in
@@ -302,17 +371,26 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
     }
   };
 
-  // LDS byte offsets (within a stage / slot) of this lane's operands
+  // LDS byte offsets (within a stage / slot) of this lane's operands.  K order
+  // of substep s: half h holds K 32h + 8s .. +7 of the step; G32: K 32(s/2) +
+  // 16h + 8(s%2) .., so that substeps 0, 1 cover the step's first group and
+  // 2, 3 its second
   int aread[4];  // A fragment of substep s of m-tile 0 (+ 32*128*mt)
 #pragma unroll
-  for (int s = 0; s < 4; ++s) aread[s] = l32 * 128 + 16 * ((4 * h + s) ^ ((l32 >> 1) & 7));
-  // codes of weight tile 0 (tile 1: rows 32 further, + 2048 bytes): 4-bit,
-  // step parity p (part 2p + h); 8-bit, half p (part 2h + p)
-  int bread[2];
+  for (int s = 0; s < 4; ++s) {
+    const int c = G32 ? 4 * (s >> 1) + 2 * h + (s & 1) : 4 * h + s;
+    aread[s] = l32 * 128 + 16 * (c ^ ((l32 >> 1) & 7));
+  }
+  // codes of weight tile 0 (tile 1: rows 32 further).  4-bit, step parity p:
+  // part 2p + h (16 bytes), G32 8 bytes at half h of part 2p + group; 8-bit,
+  // half p: part 2h + p (G32: group p, part 2p + h); 6-bit: 24 bytes at 24h
+  // (G32: 12 bytes at 12h of the group's 24)
+  int bread[4];
 #pragma unroll
-  for (int p = 0; p < 2; ++p) {
-    const int part = BITS == 4 ? 2 * p + h : 2 * h + p;
-    bread[p] = l32 * kChunkRow + 16 * (part ^ ((l32 >> 2) & 3));
+  for (int p = 0; p < 4; ++p) {
+    if constexpr (BITS == 4 && G32) bread[p] = l32 * kChunkRow + 16 * (p ^ ((l32 >> 2) & 3)) + 8 * h;
+    else if constexpr (BITS == 6) bread[p] = l32 * kChunkRow + (G32 ? 12 : 24) * h;
+    else bread[p] = l32 * kChunkRow + 16 * (((BITS == 4 || G32 ? 2 * p + h : 2 * h + p) & 3) ^ ((l32 >> 2) & 3));
   }
 
   f32x16 acc[MT][2];
@@ -390,8 +468,8 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
   //      (its loads overlap the pipeline fill) ----
   {
     // round 0 has landed: only the loads issued after it may be in flight
-    if (a.wide_scales) wait_vmcnt<1 + 4 + kLead * MT>();
-    else wait_vmcnt<4 + 4 + kLead * MT>();
+    if (a.wide_scales) wait_vmcnt<1 + kBI + kLead * MT>();
+    else wait_vmcnt<4 + kBI + kLead * MT>();
     const bool has_b = a.b[0] != nullptr;
     for (int c = 0; c < a.nch; ++c) {
       if ((c & 1) == 0) {
@@ -447,27 +525,31 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
     }
   }
 
-  // step 0's tiles and the scales have landed (4-bit: step 1's activations may
-  // still be in flight)
-  wait_vmcnt<BITS == 4 ? MT : 0>();
+  // step 0's tiles and the scales have landed (4, 6 bits: step 1's activations
+  // may still be in flight)
+  wait_vmcnt<BITS == 8 ? 0 : MT>();
   lds_barrier();
 
   const uint32_t k4300 = 0x43004300u;
-  const int sc_period = 8 * gdiv;  // K steps per 8-group scale chunk
+  const int sc_period = G32 ? 4 : 8 * gdiv;  // K steps per 8-group scale chunk
   // per-step indices carried from step to step (a runtime division by gdiv
   // or sc_period costs about 15 scalar instructions a step): the step's
   // group g and its K step within the group, the steps since the last scale
   // chunk load, the activation stages of this step and of step ks + kLead
   int g = 0, g_step = 0, sc_step = 0, sc_chunk = 0, stage = 0, stage_lead = kLead % kAStages;
   for (int ks = 0; ks < KS; ++ks) {
-    // ---- scale of the step's group for both weight tiles ----
+    // ---- scale of the step's group for both weight tiles (G32: of its two
+    //      groups, the halves of one dword) ----
     const int gi = g - max(min(8 * (g >> 3), G - 8), 0);
     const uint32_t sd = gi < 2 ? sc_cur[0] : gi < 4 ? sc_cur[1] : gi < 6 ? sc_cur[2] : sc_cur[3];
     const auto ss = __builtin_amdgcn_permlane32_swap(sd, sd, false, false);  // [nt]: tile nt's row
     const bool odd = gi & 1;
-    float sc[2];
+    float sc[2], sc1[2];
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) sc[nt] = __uint_as_float(odd ? (ss[nt] & 0xffff0000u) : (ss[nt] << 16));
+    for (int nt = 0; nt < 2; ++nt) {
+      sc[nt] = __uint_as_float(!G32 && odd ? (ss[nt] & 0xffff0000u) : (ss[nt] << 16));
+      sc1[nt] = __uint_as_float(ss[nt] & 0xffff0000u);  // (G32)
+    }
 
     // ---- loads for later steps: after the last step of a scale chunk, the
     //      next chunk into the same registers (issued first: the end-of-step
@@ -477,7 +559,7 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
       sc_step = 0;
       if (ks + 1 < KS) load_sc(++sc_chunk, sc_cur);
     }
-    if constexpr (BITS == 4) {
+    if constexpr (BITS != 8) {
       // at the first step of a code chunk the next chunk, first; then the
       // activations kLead steps ahead.  Past the end these re-read the last
       // step's tiles / chunk into a stage / slot that no later step reads, so
@@ -495,13 +577,39 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
     bf16x8 bf[2][4];
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
+      const uint8_t* ct = cb + 32 * kChunkRow * nt;
       if constexpr (BITS == 4) {
-        const u32x4 c = *reinterpret_cast<const u32x4*>(cb + bread[ks & 1] + 2048 * nt);
+        u32x4 c;
+        if constexpr (G32) {
+          const u32x2 lo = *reinterpret_cast<const u32x2*>(ct + bread[2 * (ks & 1)]);
+          const u32x2 hi = *reinterpret_cast<const u32x2*>(ct + bread[2 * (ks & 1) + 1]);
+          c = u32x4{lo.x, lo.y, hi.x, hi.y};
+        } else {
+          c = *reinterpret_cast<const u32x4*>(ct + bread[ks & 1]);
+        }
 #pragma unroll
         for (int s = 0; s < 4; ++s) bf[nt][s] = PAIRS ? expand_q4_pairs(c[s], k4300) : expand_q4(c[s], k4300);
+      } else if constexpr (BITS == 6) {
+        uint32_t d[6];
+        if constexpr (G32) {
+#pragma unroll
+          for (int i = 0; i < 6; ++i)
+            d[i] = *reinterpret_cast<const uint32_t*>(ct + bread[0] + (i < 3 ? 4 * i : 24 + 4 * (i - 3)));
+        } else {
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            const u32x2 v = *reinterpret_cast<const u32x2*>(ct + bread[0] + 8 * i);
+            d[2 * i] = v.x;
+            d[2 * i + 1] = v.y;
+          }
+        }
+        bf[nt][0] = expand_q6<PAIRS, 0>(d, k4300);
+        bf[nt][1] = expand_q6<PAIRS, 1>(d, k4300);
+        bf[nt][2] = expand_q6<PAIRS, 2>(d, k4300);
+        bf[nt][3] = expand_q6<PAIRS, 3>(d, k4300);
       } else {
-        const u32x4 c0 = *reinterpret_cast<const u32x4*>(cb + bread[0] + 2048 * nt);
-        const u32x4 c1 = *reinterpret_cast<const u32x4*>(cb + bread[1] + 2048 * nt);
+        const u32x4 c0 = *reinterpret_cast<const u32x4*>(ct + bread[0]);
+        const u32x4 c1 = *reinterpret_cast<const u32x4*>(ct + bread[1]);
         bf[nt][0] = expand_q8<PAIRS>(c0[0], c0[1]);
         bf[nt][1] = expand_q8<PAIRS>(c0[2], c0[3]);
         bf[nt][2] = expand_q8<PAIRS>(c1[0], c1[1]);
@@ -519,6 +627,20 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
 #pragma unroll
       for (int s = 0; s < 4; ++s)
         af[s] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(sa + mt * 32 * 128 + aread[s]));
+      if constexpr (G32) {  // a chain of two MFMAs and a fold per group
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+#pragma unroll
+          for (int nt = 0; nt < 2; ++nt) {
+            f32x16 p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[2 * q], bf[nt][2 * q], zero, 0, 0, 0);
+            p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[2 * q + 1], bf[nt][2 * q + 1], p, 0, 0, 0);
+            const float s = q ? sc1[nt] : sc[nt];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[mt][nt][r] = __builtin_fmaf(s, p[r], acc[mt][nt][r]);
+          }
+        }
+        continue;
+      }
       f32x16 p0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[0], bf[0][0], zero, 0, 0, 0);
 #pragma unroll
       for (int s = 1; s < 4; ++s) p0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[s], bf[0][s], p0, 0, 0, 0);
@@ -535,10 +657,12 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
     // only this step's activations (4-bit; its code chunk, issued before
     // them, is waited for: one step early at the first step of a chunk).
     // 8-bit runs one step ahead: nothing.
-    if constexpr (BITS == 4) wait_vmcnt<MT>();
+    if constexpr (BITS != 8) wait_vmcnt<MT>();
     else wait_vmcnt<0>();
     lds_barrier();
-    if (++g_step == gdiv) {
+    if constexpr (G32) {
+      g += 2;
+    } else if (++g_step == gdiv) {
       g_step = 0;
       ++g;
     }
@@ -558,10 +682,18 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
     const int m = tid / CPR + RPP * j;
     orow[j] = m < rows ? (a.row_out ? a.row_out[row0 + m] : row0 + m) : 0;
   }
-  const int hs_gpt = GLU && a.hsum ? OW / a.hsum_gs : 1;  // h groups per tile: 2 (gs 64) or 1 (gs 128)
-  const int hs_m = tid / hs_gpt;
-  int hs_row = 0;
-  if (GLU && a.hsum && hs_m < rows) hs_row = a.row_out ? a.row_out[row0 + hs_m] : row0 + hs_m;
+  // h groups per tile row: 4, 2 or 1 (group size 32, 64, 128); a thread takes
+  // the (row, group) pairs tid and, at four groups, tid + 256
+  const int hs_gpt = GLU && a.hsum ? OW / a.hsum_gs : 1;
+  int hs_row[2] = {0, 0};
+  if (GLU && a.hsum) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      if (i == 1 && hs_gpt < 4) break;  // (uniform)
+      const int m = (tid + kThreads * i) / hs_gpt;
+      if (m < rows) hs_row[i] = a.row_out ? a.row_out[row0 + m] : row0 + m;
+    }
+  }
 
   // ---- epilogue: the output tile goes through LDS so that global stores
   //      are 16-byte, whole-row-segment writes.  D layout of the 32x32 MFMA:
@@ -649,11 +781,15 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
   }
   if constexpr (GLU) {
     if (a.hsum) {
-      // group sums of the bf16 h values of this tile's 128 columns: one
-      // (row, group) per thread, written at the row's output index
+      // group sums of the bf16 h values of this tile's 128 columns, written at
+      // the row's output index
       const int gpt = hs_gpt;
-      const int m = hs_m, q = tid - m * gpt;
-      if (m < rows) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (i == 1 && gpt < 4) break;  // (uniform: 256 / gpt >= BM rows were taken in one round)
+        const int x = tid + kThreads * i;
+        const int m = x / gpt, q = x - m * gpt;
+        if (m >= rows) continue;
         float sum = 0.0f;
         for (int c = 0; c < a.hsum_gs; c += 8) {
           const u32x4 v = *reinterpret_cast<const u32x4*>(ot + m * OS + q * a.hsum_gs + c);
@@ -663,7 +799,7 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
             sum += __uint_as_float(v[j] & 0xffff0000u);
           }
         }
-        uint16_t* dst = a.hsum + static_cast<int64_t>(hs_row) * a.hsum_nch * 32;
+        uint16_t* dst = a.hsum + static_cast<int64_t>(hs_row[i]) * a.hsum_nch * 32;
         const int g = ntile * gpt + q;
         uint16_t hi, lo;
         split_bf16(sum, hi, lo);
@@ -688,7 +824,7 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
 // robin, so that the last workgroups to run are short ones.  The grid is sized
 // for the most tiles P rows can need; the split follows the real counts.  All
 // four bodies share the one LDS allocation (the 128-row body needs the most).
-template <int BITS, bool GLU, bool PAIRS, bool GACT = false>
+template <int BITS, bool GLU, bool PAIRS, bool GACT, bool G32>
 __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_prefill_kernel(PArgs a) {
   __shared__ __attribute__((aligned(1024))) uint8_t lds[prefill_lds_bytes<BITS, GLU, 4>()];
   const int bid = blockIdx.x;
@@ -713,13 +849,13 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_prefill_kernel(PArgs
   }
   const int4 tinfo = reinterpret_cast<const int4*>(a.tiles)[1 + slot];
   if (slot < cnt.x)
-    prefill_tile<BITS, GLU, 4, PAIRS, GACT>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+    prefill_tile<BITS, GLU, 4, PAIRS, GACT, G32>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
   else if (slot < nlong)
-    prefill_tile<BITS, GLU, 3, PAIRS, GACT>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+    prefill_tile<BITS, GLU, 3, PAIRS, GACT, G32>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
   else if (slot < nlong + cnt.z)
-    prefill_tile<BITS, GLU, 2, PAIRS, GACT>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+    prefill_tile<BITS, GLU, 2, PAIRS, GACT, G32>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
   else
-    prefill_tile<BITS, GLU, 1, PAIRS, GACT>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+    prefill_tile<BITS, GLU, 1, PAIRS, GACT, G32>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
 }
 
 // xhl[r] = the group sums X[g] (fp32) of row src(r) as bf16 hi and lo parts,
@@ -755,7 +891,7 @@ __global__ __launch_bounds__(256) void group_sums_kernel(const uint16_t* __restr
   // every lane of the wave takes part in the row sums (no lane has left)
   s += dpp_f<kDppQuadXor1>(s);
   s += dpp_f<kDppQuadXor2>(s);
-  s += dpp_f<kDppHalfMirror>(s);
+  if constexpr (L >= 8) s += dpp_f<kDppHalfMirror>(s);
   if constexpr (L == 16) s += dpp_f<kDppMirror>(s);
   if (part == 0 && r < R) {
     uint16_t hi, lo;
@@ -794,11 +930,20 @@ __global__ __launch_bounds__(1024) void make_tiles_kernel(const int32_t* __restr
                 base[3][t], base[0][E], base[1][E], base[2][E]);
 }
 
-template <int BITS, bool GLU, bool PAIRS, bool GACT = false>
+template <int BITS, bool GLU, bool PAIRS, bool GACT, bool G32>
 int launch_prefill(const PArgs& a, unsigned grid, hipStream_t stream) {
-  MOE_LAUNCH(GLU ? "gemm_gate_up_swiglu" : "gemm_down", (grouped_gemm_prefill_kernel<BITS, GLU, PAIRS, GACT>),
+  MOE_LAUNCH(GLU ? "gemm_gate_up_swiglu" : "gemm_down", (grouped_gemm_prefill_kernel<BITS, GLU, PAIRS, GACT, G32>),
              dim3(grid), dim3(kThreads), 0, stream, a);
   return launch_status("grouped_gemm_prefill");
+}
+
+template <int BITS, bool G32>
+int launch_bits(const PArgs& a, bool glu, bool pairs, unsigned grid, hipStream_t stream) {
+  if (glu)
+    return a.act != MOE_ACT_SWIGLU ? launch_prefill<BITS, true, true, true, G32>(a, grid, stream)
+                                   : launch_prefill<BITS, true, true, false, G32>(a, grid, stream);
+  return pairs ? launch_prefill<BITS, false, true, false, G32>(a, grid, stream)
+               : launch_prefill<BITS, false, false, false, G32>(a, grid, stream);
 }
 
 }  // namespace
@@ -811,8 +956,7 @@ int prefill_gsum_stride(const moe_qweight* w) { return (w->K / w->group_size + 1
 int64_t prefill_tile_ints(int64_t P, int E) { return 4 * (1 + P / 128 + 3 * std::min<int64_t>(E, P)); }
 
 bool prefill_supported(const moe_qweight* w0, const moe_qweight* w1) {
-  if (w0->bits != 4 && w0->bits != 8) return false;  // 6-bit experts: the per-16-row kernel
-  if (w0->group_size % 64 != 0) return false;
+  if (w0->bits != 4 && w0->bits != 6 && w0->bits != 8) return false;  // 2, 3, 5 bits: the per-16-row kernel
   const int G = w0->K / w0->group_size;
   if (G % 2 != 0) return false;  // scale pairs are read as aligned dwords
   // code chunks are 16-byte loads of 64-byte row segments (two K steps at 4 bits)
@@ -853,17 +997,21 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
   const bool by_pos = x_rows < 0;
   const int64_t R = by_pos ? P : x_rows;
   if (R > 0 && !(pf.gsum_ready && !by_pos)) {
-    const int L = w0->group_size / 8;  // 8 or 16 lanes per group
+    const int L = w0->group_size / 8;  // 4, 8 or 16 lanes per group
+    uint16_t* xp = w1 && !pf.xp_ready ? pf.xp : nullptr;
     const int64_t threads = R * (gstride / 16) * 16 * L;
     if ((threads + 255) / 256 > 0x7fffffffLL) return MOE_E_UNSUPPORTED;
     const dim3 grid(static_cast<unsigned>((threads + 255) / 256));
     const int32_t* rin = by_pos ? row_in : nullptr;
-    if (L == 8)
+    if (L == 4)
+      MOE_LAUNCH("group_sums", group_sums_kernel<4>, grid, dim3(256), 0, stream, x, rin, R, w0->K, gstride / 16,
+                 reinterpret_cast<uint16_t*>(gsum), xp);
+    else if (L == 8)
       MOE_LAUNCH("group_sums", group_sums_kernel<8>, grid, dim3(256), 0, stream, x, rin, R, w0->K, gstride / 16,
-                 reinterpret_cast<uint16_t*>(gsum), w1 ? pf.xp : nullptr);
+                 reinterpret_cast<uint16_t*>(gsum), xp);
     else
       MOE_LAUNCH("group_sums", group_sums_kernel<16>, grid, dim3(256), 0, stream, x, rin, R, w0->K, gstride / 16,
-                 reinterpret_cast<uint16_t*>(gsum), w1 ? pf.xp : nullptr);
+                 reinterpret_cast<uint16_t*>(gsum), xp);
     MOE_CHECK_LAUNCH("group_sums");
   }
   if (!pf.tiles_ready) {
@@ -915,13 +1063,12 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
   const int64_t grid = 8 * ((((P / 128 + slots) * nt + 7) / 8) + (2 * slots * nt + 7) / 8);
   if (grid > 0x7fffffffLL) return MOE_E_UNSUPPORTED;
   const unsigned g = static_cast<unsigned>(grid);
-  const bool gact = a.act != MOE_ACT_SWIGLU;
-  if (w0->bits == 4) {
-    if (w1) return gact ? launch_prefill<4, true, true, true>(a, g, stream) : launch_prefill<4, true, true>(a, g, stream);
-    return pf.in_p8 ? launch_prefill<4, false, true>(a, g, stream) : launch_prefill<4, false, false>(a, g, stream);
-  }
-  if (w1) return gact ? launch_prefill<8, true, true, true>(a, g, stream) : launch_prefill<8, true, true>(a, g, stream);
-  return pf.in_p8 ? launch_prefill<8, false, true>(a, g, stream) : launch_prefill<8, false, false>(a, g, stream);
+  const bool g32 = a.gs == 32;
+  if (w0->bits == 4)
+    return g32 ? launch_bits<4, true>(a, w1, pf.in_p8, g, stream) : launch_bits<4, false>(a, w1, pf.in_p8, g, stream);
+  if (w0->bits == 6)
+    return g32 ? launch_bits<6, true>(a, w1, pf.in_p8, g, stream) : launch_bits<6, false>(a, w1, pf.in_p8, g, stream);
+  return g32 ? launch_bits<8, true>(a, w1, pf.in_p8, g, stream) : launch_bits<8, false>(a, w1, pf.in_p8, g, stream);
 }
 
 }  // namespace moe

@@ -298,15 +298,26 @@ def test_gather_qmm_large_buckets(bits, E, N, K, batch, skew, gs):
     assert_close(hbf(got), ref, what="gather_qmm (large buckets)")
 
 
+@pytest.mark.parametrize("bits,gs,K", [(6, 64, 64 * 10), (6, 128, 512), (6, 32, 192), (4, 32, 640), (8, 32, 192)])
+def test_gather_qmm_tile_classes_widths(bits, gs, K):
+    """Both ends of every token-tile class on the large-bucket GEMM's other operand layouts (6-bit codes,
+    groups of 32), at group counts that are and are not multiples of the 8 a scale load covers."""
+    _tile_classes_case(bits, gs, K)
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 def test_gather_qmm_tile_classes(bits):
     """Bucket remainders (mod 128 rows) of 0, 1, 32, 33, 64, 65, 96, 97 and 127
     rows: every token-tile class of the large-bucket GEMM (128-row tiles, and
     remainder tiles of 32, 64, 96 and a partial 128 rows, each at both ends of
     its range)."""
+    _tile_classes_case(bits, 64, 512)
+
+
+def _tile_classes_case(bits, gs, K):
     counts = [128, 129, 160, 161, 192, 193, 224, 225, 255]
-    E, N, K = len(counts), 256, 512
-    q = W.make_qweight(bits + 30, 2, E, N, K, 0.02, 64, bits)
+    E, N = len(counts), 256
+    q = W.make_qweight(bits + 30, 2, E, N, K, 0.02, gs, bits)
     rhs = np.repeat(np.arange(E, dtype=np.uint32), counts)
     batch = rhs.size
     rng = np.random.default_rng(11)
@@ -479,6 +490,14 @@ def test_switch_glu(T, k, E, H, I, bits, gs):
     """SwitchGLU (switch_layers.cpp:200-245) against the checker's composition of the
     reference ops: gather_qmm(gate), gather_qmm(up), swiglu, gather_qmm(down), unsorted."""
     _switch_glu_case(T, k, E, H, I, bits, gs, False)
+
+
+@pytest.mark.parametrize("T,k,E,H,I,bits,gs", [(300, 2, 4, 512, 256, 6, 64), (300, 2, 4, 512, 256, 6, 32),
+                                               (301, 2, 4, 256, 768, 4, 32), (77, 2, 2, 512, 256, 8, 32)])
+def test_switch_glu_large_buckets_widths(T, k, E, H, I, bits, gs):
+    """gate|up and down on the large-bucket GEMM with 6-bit codes and with groups of 32 (gate|up then
+    writes four group sums of h per 128 columns, for 24 groups a row at I = 768: not a multiple of 16)."""
+    _switch_glu_case(T, k, E, H, I, bits, gs, True)
 
 
 @pytest.mark.parametrize("T,k,E,H,I,bits", [(16, 2, 8, 512, 1024, 4), (600, 2, 4, 512, 256, 4), (40, 4, 6, 256, 512, 8)])
