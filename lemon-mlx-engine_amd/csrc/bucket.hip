@@ -40,14 +40,14 @@ __global__ __launch_bounds__(NW * 64) void bucket_fused_kernel(const uint32_t* _
 
 __global__ __launch_bounds__(256) void bucket_count_kernel(const uint32_t* __restrict__ inds,
                                                           int64_t P, int E,
-                                                          int* __restrict__ cnt, int chunk) {
+                                                          int* __restrict__ cnt, int chunk, BucketOut o) {
   extern __shared__ int hist[];
   for (int x = threadIdx.x; x < E; x += 256) hist[x] = 0;
   __syncthreads();
   const int64_t b0 = static_cast<int64_t>(blockIdx.x) * chunk;
   const int64_t b1 = b0 + chunk < P ? b0 + chunk : P;
   for (int64_t i = b0 + threadIdx.x; i < b1; i += 256) {
-    const uint32_t v = inds[i];
+    const uint32_t v = pair_expert(inds, i, P, E, o);
     if (v < static_cast<uint32_t>(E)) atomicAdd(&hist[v], 1);
   }
   __syncthreads();
@@ -60,13 +60,12 @@ __global__ __launch_bounds__(256) void bucket_count_kernel(const uint32_t* __res
 // sums chunks [part*L, part*L + L) of expert e, the PARTS partial sums of an
 // expert are scanned through LDS, and each thread writes its range's starts.
 template <bool STAGED>
-__global__ __launch_bounds__(1024) void bucket_scan_kernel(int* __restrict__ cnt, int nblk, int E,
+__global__ __launch_bounds__(1024) void bucket_scan_kernel(int* __restrict__ cnt, int nblk, int64_t P, int E,
                                                           BucketOut o) {
   extern __shared__ int lds[];
   int* tot = lds;           // [E]
   int* offs = tot + E;      // [E+1]
-  int* tmp = offs + E + 1;  // [16 + 2]
-  int* psum = tmp + 18;     // [1024]: partial sums, [part][E]
+  int* psum = offs + E + 1; // [1024]: partial sums, [part][E]
   int* tab = psum + 1024;   // [nblk * E] (STAGED)
   const int n = nblk * E;
   if constexpr (STAGED) {  // every load of a thread in flight before its LDS stores
@@ -97,7 +96,7 @@ __global__ __launch_bounds__(1024) void bucket_scan_kernel(int* __restrict__ cnt
     tot[x] = t;
   }
   __syncthreads();
-  finish_offsets<1024>(tot, E, offs, tmp, o);
+  finish_offsets<1024>(tot, P, E, offs, o);
   if (mine) {
     int run = offs[e];
     for (int q = 0; q < part; ++q) run += psum[q * E + e];
@@ -122,8 +121,10 @@ __global__ __launch_bounds__(256) void bucket_scatter_kernel(const uint32_t* __r
   __syncthreads();
   const int64_t b0 = static_cast<int64_t>(blockIdx.x) * kChunk;
   const int64_t b1 = b0 + kChunk < P ? b0 + kChunk : P;
-  for (int64_t first = b0; first < b1; first += 256)
-    scatter_subchunk<4>(inds, b1, first, E, k, nbits, running, wcnt, o);
+  for (int64_t first = b0; first < b1; first += 256) {
+    const int64_t i = first + threadIdx.x;
+    scatter_subchunk<4>(pair_expert(inds, i, b1, E, o), i, b1, E, k, nbits, running, wcnt, o, first + 256 >= b1);
+  }
 }
 
 // Scan and scatter in one launch: workgroup b forms the per-expert totals,
@@ -133,7 +134,7 @@ __global__ __launch_bounds__(256) void bucket_scatter_kernel(const uint32_t* __r
 // so the order does not matter), then scatters chunk b.  Workgroup 0 also
 // writes offsets, the slot records and the token-tile table.  The positions
 // are those of bucket_scan_kernel + bucket_scatter_kernel.  1024 threads,
-// E <= kScanScatterMaxE; lds: 2048 + 2E + 1 + 18 + 16E ints.
+// E <= kScanScatterMaxE; lds: 2048 + 2E + 1 + 16E ints.
 __global__ __launch_bounds__(1024) void bucket_scan_scatter_kernel(const uint32_t* __restrict__ inds, int64_t P,
                                                                   int E, int k, int nbits,
                                                                   const int* __restrict__ cnt, int nblk,
@@ -143,9 +144,11 @@ __global__ __launch_bounds__(1024) void bucket_scan_scatter_kernel(const uint32_
   int* ppre = ptot + 1024;      // [parts][E]: partial counts before chunk b (row 0: the sums)
   int* tot = ppre + 1024;       // [E]
   int* running = tot + E;       // [E+1]
-  int* tmp = running + E + 1;   // [16 + 2]
-  int* wcnt = tmp + 18;         // [16][E]
+  int* wcnt = running + E + 1;  // [16][E]
   const int b = blockIdx.x;
+  const int64_t c0 = static_cast<int64_t>(b) * kFusedChunk;
+  const int64_t c1 = c0 + kFusedChunk < P ? c0 + kFusedChunk : P;
+  const uint32_t ex = pair_expert(inds, c0 + threadIdx.x, c1, E, o);  // this thread's pair (read ahead of the scan)
   const int parts = 1024 / E;
   const int L = (nblk + parts - 1) / parts;
   const int e = threadIdx.x % E, part = threadIdx.x / E;
@@ -180,13 +183,12 @@ __global__ __launch_bounds__(1024) void bucket_scan_scatter_kernel(const uint32_
     head.active = nullptr;
     head.num_active = nullptr;
     head.tiles = nullptr;
+    head.in_rows = nullptr;
   }
-  finish_offsets<1024>(tot, E, running, tmp, head);
+  finish_offsets<1024>(tot, P, E, running, head);
   for (int x = threadIdx.x; x < E; x += 1024) running[x] += ppre[x];
   __syncthreads();
-  const int64_t c0 = static_cast<int64_t>(b) * kFusedChunk;
-  const int64_t c1 = c0 + kFusedChunk < P ? c0 + kFusedChunk : P;
-  scatter_subchunk<16>(inds, c1, c0, E, k, nbits, running, wcnt, o);
+  scatter_subchunk<16>(ex, c0 + threadIdx.x, c1, E, k, nbits, running, wcnt, o, true);
 }
 
 }  // namespace
@@ -207,7 +209,7 @@ int bucket(const uint32_t* inds, int64_t T, int k, int E, const BucketOut& o, vo
   const int nbits = bits_for(E);
   if (P <= kFusedMaxP && E <= kFusedMaxE) {
     constexpr int NW = 16;
-    const size_t lds = sizeof(int) * bucket_fused_lds_ints<NW>(E);
+    const size_t lds = sizeof(int) * bucket_fused_lds_ints<NW>(E, P);
     MOE_LAUNCH("bucket_fused", bucket_fused_kernel<NW>, dim3(1), dim3(NW * 64), lds, stream, inds, P, E,
                        k, nbits, o);
     MOE_CHECK_LAUNCH("bucket_fused");
@@ -221,23 +223,23 @@ int bucket(const uint32_t* inds, int64_t T, int k, int E, const BucketOut& o, vo
     // (the table of 1024-pair chunks is at most half the workspace's 512-pair one)
     const int nb = static_cast<int>(nblk_f);
     MOE_LAUNCH("bucket_count", bucket_count_kernel, dim3(nb), dim3(256), sizeof(int) * E, stream, inds, P, E, cnt,
-               kFusedChunk);
+               kFusedChunk, o);
     MOE_CHECK_LAUNCH("bucket_count");
     MOE_LAUNCH("bucket_scatter", bucket_scan_scatter_kernel, dim3(nb), dim3(1024),
-               sizeof(int) * (2048 + 2 * E + 1 + 18 + 16 * E), stream, inds, P, E, k, nbits, cnt, nb, o);
+               sizeof(int) * (2048 + 2 * E + 1 + 16 * E), stream, inds, P, E, k, nbits, cnt, nb, o);
     MOE_CHECK_LAUNCH("bucket_scatter");
     return MOE_OK;
   }
   const int nblk = static_cast<int>((P + kChunk - 1) / kChunk);
   MOE_LAUNCH("bucket_count", bucket_count_kernel, dim3(nblk), dim3(256), sizeof(int) * E, stream, inds, P,
-                     E, cnt, kChunk);
+                     E, cnt, kChunk, o);
   MOE_CHECK_LAUNCH("bucket_count");
   if (static_cast<int64_t>(nblk) * E <= kScanStagedMax)
     MOE_LAUNCH("bucket_scan", bucket_scan_kernel<true>, dim3(1), dim3(1024),
-               sizeof(int) * (2 * E + 1 + 18 + 1024 + nblk * E), stream, cnt, nblk, E, o);
+               sizeof(int) * (2 * E + 1 + 1024 + nblk * E), stream, cnt, nblk, P, E, o);
   else
-    MOE_LAUNCH("bucket_scan", bucket_scan_kernel<false>, dim3(1), dim3(1024), sizeof(int) * (2 * E + 1 + 18 + 1024),
-               stream, cnt, nblk, E, o);
+    MOE_LAUNCH("bucket_scan", bucket_scan_kernel<false>, dim3(1), dim3(1024), sizeof(int) * (2 * E + 1 + 1024),
+               stream, cnt, nblk, P, E, o);
   MOE_CHECK_LAUNCH("bucket_scan");
   MOE_LAUNCH("bucket_scatter", bucket_scatter_kernel, dim3(nblk), dim3(256), sizeof(int) * 5 * E, stream,
                      inds, P, E, k, nbits, cnt, o);

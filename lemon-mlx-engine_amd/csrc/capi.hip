@@ -64,33 +64,6 @@ __global__ void fill_shared_meta(int32_t* offsets, int32_t* active, int32_t* num
   }
 }
 
-// pair i = (b, m) takes expert rhs[b].  A pair whose expert is out of range
-// is left out by the bucketing; its output row (row i of out [*, N]) is
-// written as zeros here so that it never returns stale memory.
-__global__ void expand_pairs(const uint32_t* __restrict__ rhs, int64_t batch, int M, int E,
-                             uint32_t* __restrict__ pair_expert, uint16_t* __restrict__ out, int N) {
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= batch * M) return;
-  const uint32_t e = rhs[i / M];
-  pair_expert[i] = e;
-  if (e >= static_cast<uint32_t>(E))
-    for (int c = 0; c < N; ++c) out[i * N + c] = 0;
-}
-
-__global__ void make_in_rows(const int32_t* __restrict__ perm, const uint32_t* __restrict__ lhs,
-                             int64_t n, int M, int32_t* __restrict__ in_rows) {
-  const int64_t pos = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (pos >= n) return;
-  const int64_t f = perm[pos];
-  if (f < 0 || f >= n) {  // a position past the buckets (pairs of out-of-range experts): never read
-    in_rows[pos] = 0;
-    return;
-  }
-  const int64_t b = f / M, m = f % M;
-  const int64_t src = lhs ? static_cast<int64_t>(lhs[b]) : b;
-  in_rows[pos] = static_cast<int32_t>(src * M + m);
-}
-
 struct BlockPlan {
   uint16_t* logits;
   uint32_t* inds;
@@ -417,12 +390,21 @@ int moe_bucket(const uint32_t* inds, int64_t T, int32_t k, int32_t E, int32_t* p
                      reinterpret_cast<hipStream_t>(stream));
 }
 
-static moe::Carve gqmm_layout(void* ws, int64_t n, int32_t E, int32_t gstride, uint32_t** pair_expert,
-                              int32_t** perm, int32_t** offsets, int32_t** active,
-                              int32_t** num_active, int32_t** in_rows, int32_t** tiles, float** gsum,
-                              char** bws, size_t* bws_bytes) {
+// The bucketing of gather_qmm's and gather_mm's pairs also writes each sorted
+// position's input row and zeroes the output rows of out-of-range experts (two
+// launches fewer).
+static void set_gather_pairs(BucketOut& o, const uint32_t* lhs, int32_t M, int32_t* in_rows, uint16_t* out, int N) {
+  o.M = M;
+  o.lhs = lhs;
+  o.in_rows = in_rows;
+  o.zero_out = out;
+  o.zero_N = N;
+}
+
+static moe::Carve gqmm_layout(void* ws, int64_t n, int32_t E, int32_t gstride, int32_t** perm, int32_t** offsets,
+                              int32_t** active, int32_t** num_active, int32_t** in_rows, int32_t** tiles,
+                              float** gsum, char** bws, size_t* bws_bytes) {
   moe::Carve c(ws);
-  *pair_expert = c.take<uint32_t>(n);
   *perm = c.take<int32_t>(n);
   *offsets = c.take<int32_t>(E + 1);
   *active = c.take<int32_t>(4 * static_cast<int64_t>(E));
@@ -442,12 +424,11 @@ constexpr int32_t kGqmmMaxGstride = 256;
 
 size_t moe_gather_qmm_workspace_size(int64_t batch, int32_t M, int32_t num_experts) {
   if (batch < 0 || M <= 0 || num_experts <= 0) return 0;
-  uint32_t* pe;
   int32_t *perm, *offs, *act, *na, *inr, *tiles;
   float* gsum;
   char* bws;
   size_t bb;
-  return gqmm_layout(nullptr, batch * M, num_experts, kGqmmMaxGstride, &pe, &perm, &offs, &act, &na, &inr,
+  return gqmm_layout(nullptr, batch * M, num_experts, kGqmmMaxGstride, &perm, &offs, &act, &na, &inr,
                      &tiles, &gsum, &bws, &bb)
       .size();
 }
@@ -466,37 +447,29 @@ int moe_gather_qmm(const uint16_t* x, const moe_qweight* w, const uint32_t* lhs,
   const size_t need = moe_gather_qmm_workspace_size(batch, M, w->experts);
   if (!workspace || workspace_bytes < need) return MOE_E_WORKSPACE;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  uint32_t* pe;
   int32_t *perm, *offs, *act, *na, *inr, *tiles;
   float* gsum;
   char* bws;
   size_t bb;
-  gqmm_layout(workspace, n, w->experts, kGqmmMaxGstride, &pe, &perm, &offs, &act, &na, &inr, &tiles, &gsum,
+  gqmm_layout(workspace, n, w->experts, kGqmmMaxGstride, &perm, &offs, &act, &na, &inr, &tiles, &gsum,
               &bws, &bb);
-  const unsigned nb = static_cast<unsigned>((n + 255) / 256);
-  MOE_LAUNCH("expand_pairs", moe::expand_pairs, dim3(nb), dim3(256), 0, s, rhs, batch, M, w->experts, pe, out,
-             w->N);
-  MOE_CHECK_LAUNCH("gather_qmm.expand");
   const int slots = static_cast<int>(n < w->experts ? n : w->experts);
   const bool pf_ok = moe::prefill_gsum_stride(w) <= kGqmmMaxGstride;
   BucketOut o{perm, nullptr, nullptr, nullptr, offs, act, na};
   // the bucketing also writes the large-bucket GEMM's token-tile table
   const bool pf_tiles = pf_ok && moe::use_prefill(n, slots, w, nullptr);
   if (pf_tiles) o.tiles = tiles;
-  st = moe::bucket(pe, n, 1, w->experts, o, bws, bb, s);
+  set_gather_pairs(o, lhs, M, inr, out, w->N);
+  st = moe::bucket(rhs, n, 1, w->experts, o, bws, bb, s);
   if (st != MOE_OK) return st;
-  MOE_LAUNCH("make_in_rows", moe::make_in_rows, dim3(nb), dim3(256), 0, s, perm, lhs, n, M, inr);
-  MOE_CHECK_LAUNCH("gather_qmm.rows");
   moe::PrefillScratch pf{tiles, gsum, -1};
   pf.tiles_ready = pf_tiles;
   return moe::grouped_qmm(x, inr, perm, offs, act, na, slots, n, pf_ok ? &pf : nullptr, w, nullptr, out, s);
 }
 
-static moe::Carve gmm_layout(void* ws, int64_t n, int32_t E, uint32_t** pair_expert, int32_t** perm,
-                             int32_t** offsets, int32_t** in_rows, int32_t** tiles, char** bws,
-                             size_t* bws_bytes) {
+static moe::Carve gmm_layout(void* ws, int64_t n, int32_t E, int32_t** perm, int32_t** offsets, int32_t** in_rows,
+                             int32_t** tiles, char** bws, size_t* bws_bytes) {
   moe::Carve c(ws);
-  *pair_expert = c.take<uint32_t>(n);
   *perm = c.take<int32_t>(n);
   *offsets = c.take<int32_t>(E + 1);
   *in_rows = c.take<int32_t>(n);
@@ -508,11 +481,10 @@ static moe::Carve gmm_layout(void* ws, int64_t n, int32_t E, uint32_t** pair_exp
 
 size_t moe_gather_mm_workspace_size(int64_t batch, int32_t M, int32_t num_experts) {
   if (batch < 0 || M <= 0 || num_experts <= 0) return 0;
-  uint32_t* pe;
   int32_t *perm, *offs, *inr, *tiles;
   char* bws;
   size_t bb;
-  return gmm_layout(nullptr, batch * M, num_experts, &pe, &perm, &offs, &inr, &tiles, &bws, &bb).size();
+  return gmm_layout(nullptr, batch * M, num_experts, &perm, &offs, &inr, &tiles, &bws, &bb).size();
 }
 
 int moe_gather_mm(const uint16_t* x, const uint16_t* w, const uint16_t* linear_bias, int32_t num_experts, int32_t N,
@@ -530,20 +502,14 @@ int moe_gather_mm(const uint16_t* x, const uint16_t* w, const uint16_t* linear_b
   const size_t need = moe_gather_mm_workspace_size(batch, M, num_experts);
   if (!workspace || workspace_bytes < need) return MOE_E_WORKSPACE;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  uint32_t* pe;
   int32_t *perm, *offs, *inr, *tiles;
   char* bws;
   size_t bb;
-  gmm_layout(workspace, n, num_experts, &pe, &perm, &offs, &inr, &tiles, &bws, &bb);
-  const unsigned nb = static_cast<unsigned>((n + 255) / 256);
-  MOE_LAUNCH("expand_pairs", moe::expand_pairs, dim3(nb), dim3(256), 0, s, rhs, batch, M, num_experts, pe, out,
-             N);
-  MOE_CHECK_LAUNCH("gather_mm.expand");
+  gmm_layout(workspace, n, num_experts, &perm, &offs, &inr, &tiles, &bws, &bb);
   BucketOut o{perm, nullptr, nullptr, nullptr, offs, nullptr, nullptr, tiles};
-  int st = moe::bucket(pe, n, 1, num_experts, o, bws, bb, s);
+  set_gather_pairs(o, lhs, M, inr, out, N);
+  const int st = moe::bucket(rhs, n, 1, num_experts, o, bws, bb, s);
   if (st != MOE_OK) return st;
-  MOE_LAUNCH("make_in_rows", moe::make_in_rows, dim3(nb), dim3(256), 0, s, perm, lhs, n, M, inr);
-  MOE_CHECK_LAUNCH("gather_mm.rows");
   const int slots = static_cast<int>(n < num_experts ? n : num_experts);
   return moe::grouped_mm(x, inr, perm, tiles, slots, n, w, linear_bias, N, K, out, s);
 }

@@ -48,6 +48,15 @@ struct BucketOut {
                            //       experts with a non-empty bucket, ascending, then rows = 0
   int32_t* num_active;     // [1]
   int32_t* tiles = nullptr;  // optional: the large-bucket GEMM's token-tile table (prefill_tile_ints)
+  // the gather_qmm / gather_mm pairs (k = 1): pair i = (b, m), b = i / M, takes
+  // expert inds[b] and input row lhs[b] * M + m (lhs NULL: row i)
+  int M = 1;
+  const uint32_t* lhs = nullptr;
+  int32_t* in_rows = nullptr;     // optional [P]: sorted position -> input row
+  // optional: row i of zero_out [P, zero_N] is zeroed for a pair whose expert
+  // is out of range (it is in no bucket, so no other kernel writes its row)
+  uint16_t* zero_out = nullptr;
+  int zero_N = 0;
 };
 
 // Group sums of x produced by the router projection for the expert GEMM

@@ -438,7 +438,7 @@ __global__ __launch_bounds__(NW * 64) void route_bucket_kernel(RouteArgs a, int 
   extern __shared__ int lds[];
   // the selected experts also go to LDS (after the bucketing's ints), so the
   // bucketing reads them without a round trip through L2
-  uint32_t* inds_lds = reinterpret_cast<uint32_t*>(lds + bucket_fused_lds_ints<NW>(a.E));
+  uint32_t* inds_lds = reinterpret_cast<uint32_t*>(lds + bucket_fused_lds_ints<NW>(a.E, a.T * a.k));
   for (int64_t t = threadIdx.x >> 6; t < a.T; t += NW) route_token<VPL>(a, t, threadIdx.x & 63, inds_lds);
   __syncthreads();  // every token's experts are written
   bucket_fused_body<NW>(inds_lds, a.T * a.k, a.E, a.k, nbits, o, lds);
@@ -764,7 +764,7 @@ int route_bucket(const uint16_t* logits, const float* bias, int64_t T, const moe
               p->norm_topk_prob, p->n_group, p->topk_group, p->routed_scaling_factor};
   constexpr int NW = 16;
   const int E = p->num_experts;
-  const size_t lds = sizeof(int) * (bucket_fused_lds_ints<NW>(E) + static_cast<size_t>(T) * p->top_k);
+  const size_t lds = sizeof(int) * (bucket_fused_lds_ints<NW>(E, T * p->top_k) + static_cast<size_t>(T) * p->top_k);
   const int nbits = bits_for(E);
   const int vpl = (E + 63) / 64;
   if (vpl <= 1)

@@ -232,6 +232,30 @@ def test_gather_mm_tiles(N, K, counts):
         assert ((got[rows] - ref).abs() <= bound).all(), f"expert {e}: {counts[e]} rows"
 
 
+@pytest.mark.parametrize("E,batch,M", [
+    (40, 150, 2), (512, 4096, 1), (40, 1365, 3),   # one workgroup buckets up to 4096 pairs, E <= 512
+    (40, 4097, 1), (40, 3000, 2),                  # count + scan-scatter
+    (600, 4500, 2), (1024, 300, 1),                # count, scan, scatter
+])
+def test_gather_pairs_bucketing(E, batch, M):
+    """Every bucketing path as gather_mm uses it: M rows per pair, gathered input rows, out-of-range experts
+    (zero rows) and empty ones.  Products of small integers, so every sum is exact."""
+    N, K = 16, 32
+    rng = np.random.default_rng(E + batch)
+    rhs = rng.integers(0, E + 1, batch).astype(np.uint32)
+    rhs[rhs == 3] = E + 7
+    lhs = rng.integers(0, 50, batch).astype(np.uint32)
+    x = torch.from_numpy(rng.integers(-4, 5, (50, M, K))).float()
+    w = torch.from_numpy(rng.integers(-2, 3, (E, N, K))).float()
+    out = torch.full((batch, M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    moe.gather_mm(x.bfloat16().to(DEV), w.bfloat16().to(DEV), di32(lhs), di32(rhs.view(np.int32)), M=M, out=out)
+    ok = torch.from_numpy(rhs < E)
+    ref = torch.zeros(batch, M, N)
+    ref[ok] = torch.matmul(x[torch.from_numpy(lhs.astype(np.int64))[ok]],
+                           w[torch.from_numpy(rhs.astype(np.int64))[ok]].transpose(1, 2)).bfloat16().float()
+    assert torch.equal(out.float().cpu(), ref)
+
+
 @pytest.mark.parametrize("kind,batch", [("q4", 16), ("q4", 1000), ("q6", 40), ("dense", 16), ("dense", 1000)])
 def test_gather_out_of_range_experts(kind, batch):
     """rhs entries >= E (outside the contract; the checker rejects them): those output rows are zeros,
