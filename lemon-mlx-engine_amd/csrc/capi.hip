@@ -86,6 +86,7 @@ struct BlockPlan {
   float* hsum;  // group sums of h (written by the gate|up GEMM for down)
   float* rpart;  // small batches: the router projection's partial sums [ks][T][E]
   int rks;       // their slice count (0: the small-batch router is not used)
+  float* sh_hsum;  // group sums of the shared expert's h, as hsum
   float* tpart;  // many tokens: the K-split projection's partial sums [tks][T][E]
   int tks;       // their slice count (1: one slice, bf16 logits straight from the projection)
 };
@@ -158,7 +159,7 @@ BlockPlan plan_block(const moe_block_desc* d, int64_t T, void* ws, size_t* total
   p.bk.offsets = c.take<int32_t>(E + 1);
   p.bk.active = c.take<int32_t>(4 * static_cast<int64_t>(E));
   p.bk.num_active = c.take<int32_t>(1);
-  p.tiles = c.take<int32_t>(moe::prefill_tile_ints(P, E));
+  p.tiles = c.take<int32_t>(moe::prefill_tile_ints(P + T, E + 1));  // (with the shared expert's T rows)
   {
     int64_t g = T * moe::prefill_gsum_stride(&d->gate);
     g = std::max<int64_t>(g, P * moe::prefill_gsum_stride(&d->down));
@@ -180,6 +181,7 @@ BlockPlan plan_block(const moe_block_desc* d, int64_t T, void* ws, size_t* total
   p.Y = c.take<uint16_t>(P * H);
   if (d->shared_intermediate > 0) {
     p.sgl = c.take<uint16_t>(T);
+    p.sh_hsum = c.take<float>(T * moe::prefill_gsum_stride(&d->shared_down));
     p.hs = c.take<uint16_t>(T * d->shared_intermediate);
     p.Ys = c.take<uint16_t>(T * H);
   }
@@ -703,7 +705,21 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   const bool rq_large = qrouter && moe::use_prefill(T, 1, &d->router_q, nullptr);
   const bool sh_up_large = d->shared_intermediate > 0 && moe::use_prefill(T, 1, &d->shared_gate, &d->shared_up);
   const bool sh_down_large = d->shared_intermediate > 0 && moe::use_prefill(T, 1, &d->shared_down, nullptr);
-  if (rq_large || sh_up_large || sh_down_large) {
+  const bool pf_up = moe::use_prefill(P, slots, &d->gate, &d->up);
+  const bool pf_down = moe::use_prefill(P, slots, &d->down, nullptr);
+  // A shared expert of the routed experts' shape runs in their launches, its T
+  // rows as one more expert's: the launches of one expert alone leave most CUs
+  // idle (Qwen3-Next T = 1001: six of them, 65 us).  Whole blocks, separate |
+  // merged (us): Qwen3-Next T = 1 36.5 | 31.1, 8 77 | 65, 128 199 | 188, 1001
+  // 389 | 346; DeepSeek-V3 T = 1 97 | 85, 64 834 | 793, 600 2074 | 1954.  On
+  // the per-16-row kernel only while the shared rows would run there too (many
+  // rows of one expert: the large-bucket GEMM by itself).
+  const bool sh_shape = d->shared_intermediate > 0 && moe::shared_fits(d->gate, d->shared_gate) &&
+                        moe::shared_fits(d->up, d->shared_up) && moe::shared_fits(d->down, d->shared_down);
+  const bool sh_large = sh_shape && pf_up && pf_down && E < 1024;
+  const bool sh_small = sh_shape && !pf_up && !pf_down && !sh_up_large && !sh_down_large;
+  const bool sh_merged = sh_large || sh_small;
+  if (rq_large || (!sh_merged && (sh_up_large || sh_down_large))) {
     MOE_LAUNCH("shared_meta", moe::fill_shared_meta, dim3(1), dim3(64), 0, s, p.sh_offsets, p.sh_active,
                p.sh_num, static_cast<int>(T));
     MOE_CHECK_LAUNCH("shared.meta");
@@ -715,10 +731,9 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
                          moe::use_prefill(P, slots, &d->gate, &d->up);
   const moe::RouterGroupSums sums{reinterpret_cast<uint16_t*>(p.gsum), d->gate.group_size,
                                   moe::prefill_gsum_stride(&d->gate) / 16};
-  const bool pf_up = moe::use_prefill(P, slots, &d->gate, &d->up);
-  const bool pf_down = moe::use_prefill(P, slots, &d->down, nullptr);
   // the bucketing also writes the large-bucket GEMM's token-tile table (one for both GEMMs)
   p.bk.tiles = pf_up || pf_down ? p.tiles : nullptr;
+  p.bk.sh_rows = sh_large ? static_cast<int>(T) : 0;
   // small batches: routing and bucketing in one workgroup, from the partial
   // sums of a router projection spread over many workgroups
   const bool small = moe::route_bucket_small_fits(T, &d->router, p.bk);
@@ -793,10 +808,18 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   // h in pair K order for a down GEMM that reads it so
   const bool h_pairs = !dc_fused && (pf_down || d->down.bits == 4);
   pf1.out_p8 = h_pairs;
+  moe::SharedRows sh1, sh2;
+  if (sh_merged) {
+    const uint16_t* sums_h = reinterpret_cast<const uint16_t*>(p.sh_hsum);
+    sh1 = {&d->shared_gate, &d->shared_up, p.xp, p.hs, reinterpret_cast<const uint16_t*>(p.gsum),
+           reinterpret_cast<uint16_t*>(p.sh_hsum), static_cast<int>(T)};
+    sh2 = {&d->shared_down, nullptr, p.hs, p.Ys, sums_h, nullptr, static_cast<int>(T)};
+    pf1.shared = &sh1;
+  }
   st = moe::grouped_qmm(x, p.bk.sorted_token, nullptr, p.bk.offsets, p.bk.active, p.bk.num_active,
                         slots, P, &pf1, &d->gate, &d->up, p.h, s);
   if (st != MOE_OK) return st;
-  if (d->shared_intermediate > 0) {
+  if (d->shared_intermediate > 0) {  // its sigmoid gate
     const moe::ProfScope scope(moe::ProfLabel::kShared);
     if (d->shared_gate_q.w) {  // linear_forward's quantized branch for the gate (qwen3_next.cpp:488)
       st = moe::qrow(x, T, &d->shared_gate_q, p.sgl, s);
@@ -805,17 +828,24 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
       st = moe::router_logits(x, d->shared_gate_weight, nullptr, T, d->hidden, 1, p.sgl, s);
       if (st != MOE_OK) return st;
     }
-    const bool sh_down = sh_down_large;
+  }
+  // the launches of its own: both projections, or (one token: down runs with
+  // the combine) its down alone
+  if (d->shared_intermediate > 0 && (!sh_merged || dc_fused)) {
+    const moe::ProfScope scope(moe::ProfLabel::kShared);
+    const bool sh_down = sh_down_large && !sh_merged;
     moe::PrefillScratch pf3{p.sh_tiles, p.gsum, T};
     pf3.xp = p.xp;
     pf3.xp_ready = !qrouter || pf_up;  // written by the bf16 router projection or by gate|up's group-sum pass
-    const bool sh_pairs = sh_down || d->shared_down.bits == 4;
+    const bool sh_pairs = sh_merged ? h_pairs : sh_down || d->shared_down.bits == 4;
     pf3.out_p8 = sh_pairs;
     pf3.gemv_only = !sh_up_large;
-    st = moe::grouped_qmm(x, nullptr, nullptr, p.sh_offsets, p.sh_active, p.sh_num,
-                          sh_up_large ? 1 : moe::one_expert_slots(T), T, &pf3, &d->shared_gate, &d->shared_up,
-                          p.hs, s);
-    if (st != MOE_OK) return st;
+    if (!sh_merged) {
+      st = moe::grouped_qmm(x, nullptr, nullptr, p.sh_offsets, p.sh_active, p.sh_num,
+                            sh_up_large ? 1 : moe::one_expert_slots(T), T, &pf3, &d->shared_gate, &d->shared_up,
+                            p.hs, s);
+      if (st != MOE_OK) return st;
+    }
     moe::PrefillScratch pf4{p.sh_tiles, p.gsum, T};
     pf4.in_p8 = sh_pairs;
     pf4.gemv_only = !sh_down;
@@ -832,6 +862,7 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   moe::PrefillScratch pf2{p.tiles, fuse_hsum ? p.hsum : p.gsum, P, fuse_hsum};
   pf2.tiles_ready = p.bk.tiles != nullptr;
   pf2.in_p8 = h_pairs;
+  if (sh_merged) pf2.shared = &sh2;
   st = moe::grouped_qmm(p.h, nullptr, p.bk.perm, p.bk.offsets, p.bk.active, p.bk.num_active, slots,
                         P, &pf2, &d->down, nullptr, p.Y, s);
   if (st != MOE_OK) return st;

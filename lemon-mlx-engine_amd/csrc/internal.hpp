@@ -48,6 +48,8 @@ struct BucketOut {
                            //       experts with a non-empty bucket, ascending, then rows = 0
   int32_t* num_active;     // [1]
   int32_t* tiles = nullptr;  // optional: the large-bucket GEMM's token-tile table (prefill_tile_ints)
+  int sh_rows = 0;  // > 0: the table also holds the tiles of the shared expert's
+                    // sh_rows rows, as one more expert, numbered -1, from row 0
   // the gather_qmm / gather_mm pairs (k = 1): pair i = (b, m), b = i / M, takes
   // expert inds[b] and input row lhs[b] * M + m (lhs NULL: row i)
   int M = 1;
@@ -164,6 +166,23 @@ struct FusedRoute {
   BucketOut o{};
 };
 
+// The shared expert run inside the routed experts' launches, as one more
+// expert over the T token rows (same shape, width and group size: see
+// shared_fits): its projections, input and output rows.  xhl / hsum: the group
+// sums of its input rows and of its h (large-bucket GEMM).
+struct SharedRows {
+  const moe_qweight* w0 = nullptr;
+  const moe_qweight* w1 = nullptr;  // gate|up
+  const uint16_t* x = nullptr;
+  uint16_t* out = nullptr;
+  const uint16_t* xhl = nullptr;
+  uint16_t* hsum = nullptr;
+  int rows = 0;
+};
+// Whether the projection s of the shared expert can run in the launch of the
+// routed projection w
+bool shared_fits(const moe_qweight& w, const moe_qweight& s);
+
 struct PrefillScratch {
   int32_t* tiles;   // [prefill_tile_ints(P, E)] token tile table
   float* gsum;      // [max(x_rows, P) * prefill_gsum_stride] 4-byte words: group sums as bf16 hi/lo planes
@@ -195,6 +214,9 @@ struct PrefillScratch {
   int act = MOE_ACT_SWIGLU;
   // gate|up at one token: route it in the kernel (gate_up_route_fits)
   const FusedRoute* route = nullptr;
+  // the shared expert in the same launch (the token-tile table then holds its
+  // tiles: BucketOut::sh_rows)
+  const SharedRows* shared = nullptr;
 };
 constexpr int kOneExpertSlots = 64;
 inline int one_expert_slots(int64_t P) { return static_cast<int>(std::min<int64_t>((P + 15) / 16, kOneExpertSlots)); }

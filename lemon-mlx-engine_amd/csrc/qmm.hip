@@ -54,6 +54,17 @@ struct GQArgs {
   int one_rows;
   int one_per;              // rows per slot: a multiple of 16
   int act;                  // GLU: moe_activation of h = act(gate, up)
+  // the shared expert: slots from sh_slot0 on, sh_per rows each of its sh_rows
+  // rows (token order), with weights, input and output rows of its own
+  int sh_slot0, sh_rows, sh_per;
+  struct Shared {
+    const uint16_t* x;
+    const uint32_t* w[2];
+    const uint16_t* s[2];
+    const uint16_t* b[2];
+    const uint16_t* lb[2];
+    uint16_t* out;
+  } sh;
   // one token routed in the kernel (RVPL > 0; see FusedRoute): the router's
   // partial sums [rks][E], its bias, and the outputs workgroup 0 writes
   const float* rpart;
@@ -264,7 +275,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PAIRS || !S
   bool valid = slot < slots;
   int e = slot;
   int beg = 0, cnt = 0;
-  if constexpr (RVPL > 0) {
+  if (valid && slot >= a.sh_slot0) {  // (RVPL: a tile per workgroup, so the whole workgroup)
+    e = 0;
+    beg = a.sh_per * (slot - a.sh_slot0);
+    cnt = min(a.sh_per, a.sh_rows - beg);
+    valid = cnt > 0;
+    a.x = a.sh.x;
+    a.row_in = nullptr;
+    a.row_out = nullptr;
+    a.out = a.sh.out;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      a.w[m] = a.sh.w[m];
+      a.s[m] = a.sh.s[m];
+      a.b[m] = a.sh.b[m];
+      a.lb[m] = a.sh.lb[m];
+    }
+  } else if constexpr (RVPL > 0) {
     // wave 0: the logits from the partial sums in its registers (slice order,
     // as route_bucket_small), the token routed, its experts sorted into the
     // slot records (the weights only in workgroup 0)
@@ -343,8 +370,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PAIRS || !S
   {
     const int mt = (sr >> 4) % NMAT;
     const int64_t row = static_cast<int64_t>(e) * a.N + min(n0 + (sr & 15), a.N - 1);
-    ssrc = a.s[mt] + row * G;
-    bsrc = a.b[mt] ? a.b[mt] + row * G : nullptr;
+    // (selects of the arguments: indexed by the lane's matrix, each lane would
+    // first load its pointers from memory)
+    const uint16_t* bm = NMAT > 1 && mt ? a.b[1] : a.b[0];
+    ssrc = (NMAT > 1 && mt ? a.s[1] : a.s[0]) + row * G;
+    bsrc = bm ? bm + row * G : nullptr;
   }
   // stage st for the batch starting at block j0: every lane issues the same
   // number of DMA instructions (3 + ROWS/8), so the wait counts are static
@@ -1190,6 +1220,29 @@ int grouped_qmm(const uint16_t* x, const int32_t* row_in, const int32_t* row_out
   a.out = out;
   a.act = w1 && pf ? pf->act : MOE_ACT_SWIGLU;
 
+  int total = slots;  // with the shared expert's
+  a.sh_slot0 = 0x7fffffff;
+  if (pf && pf->shared) {
+    const SharedRows& sh = *pf->shared;
+    if (!sh.w0 || !sh.x || !sh.out || sh.rows < 1 || (w1 != nullptr) != (sh.w1 != nullptr) || pf->gemv_only ||
+        !shared_fits(*w0, *sh.w0) || (w1 && !shared_fits(*w1, *sh.w1)) || (reinterpret_cast<uintptr_t>(sh.x) & 15u))
+      return MOE_E_INVALID_ARG;
+    const int n = one_expert_slots(sh.rows);
+    a.sh_slot0 = slots;
+    a.sh_rows = sh.rows;
+    a.sh_per = (sh.rows + n - 1) / n;
+    a.sh_per = (a.sh_per + 15) / 16 * 16;
+    a.sh.x = w1 ? a.x : sh.x;  // gate|up: the token rows the routed experts gather from
+    a.sh.out = sh.out;
+    const moe_qweight* sw[2] = {sh.w0, sh.w1 ? sh.w1 : sh.w0};
+    for (int m = 0; m < 2; ++m) {
+      a.sh.w[m] = sw[m]->w;
+      a.sh.s[m] = sw[m]->scales;
+      a.sh.b[m] = sw[m]->biases;
+      a.sh.lb[m] = sw[m]->linear_bias;
+    }
+    total += n;
+  }
   const int ksplit = gqmm_ksplit(P, slots, w0);
   // 2, 3 and 5 bits, and group size 32: one tile per wave, scales staged with the codes
   const bool plain = w0->bits == 2 || w0->bits == 3 || w0->bits == 5 || w0->group_size == 32;
@@ -1202,11 +1255,16 @@ int grouped_qmm(const uint16_t* x, const int32_t* row_in, const int32_t* row_out
     a.w[1] = w0->w + rows16 * w0->K * w0->bits / 32;
     a.s[1] = w0->scales + rows16 * (w0->K / w0->group_size);
     a.b[1] = w0->biases ? w0->biases + rows16 * (w0->K / w0->group_size) : nullptr;
+    if (total > slots) {
+      a.sh.w[1] = a.sh.w[0] + rows16 * w0->K * w0->bits / 32;
+      a.sh.s[1] = a.sh.s[0] + rows16 * (w0->K / w0->group_size);
+      a.sh.b[1] = a.sh.b[0] ? a.sh.b[0] + rows16 * (w0->K / w0->group_size) : nullptr;
+    }
   }
   const bool roll = !plain && part_groups(w0->K, w0->bits, w0->group_size, ksplit) > 32;
   const int mode = duo ? (sreg ? (roll ? 5 : 4) : 2) : sreg && w1 ? (roll ? 3 : 1) : 0;
   const int tiles16 = duo ? a.N / 32 : (a.N + 15) / 16;  // tiles of one wave (per K part)
-  const int64_t tiles = static_cast<int64_t>(tiles16) * slots;
+  const int64_t tiles = static_cast<int64_t>(tiles16) * total;
   if (tiles > 0x7fffffffLL) return MOE_E_UNSUPPORTED;
   if (pf && pf->route) {  // one token, routed by the gate|up kernel itself
     const FusedRoute& fr = *pf->route;
@@ -1221,29 +1279,29 @@ int grouped_qmm(const uint16_t* x, const int32_t* row_in, const int32_t* row_out
     a.ra = RouteArgs{nullptr, fr.score_bias, fr.inds, fr.scores, 1, rp.num_experts, rp.top_k, rp.variant,
                      rp.norm_topk_prob, rp.n_group, rp.topk_group, rp.routed_scaling_factor};
     a.rbo = fr.o;
-    return a.gs == 64 ? launch_routed<64>(a, tiles16, slots, stream) : launch_routed<128>(a, tiles16, slots, stream);
+    return a.gs == 64 ? launch_routed<64>(a, tiles16, total, stream) : launch_routed<128>(a, tiles16, total, stream);
   }
   if (w0->bits == 4) {
     if (pairs)
-      return w1 ? launch_gs<4, true, true>(a, ksplit, mode, tiles16, slots, stream)
-                : launch_gs<4, false, true>(a, ksplit, mode, tiles16, slots, stream);
-    return w1 ? launch_gs<4, true, false>(a, ksplit, mode, tiles16, slots, stream)
-              : launch_gs<4, false, false>(a, ksplit, mode, tiles16, slots, stream);
+      return w1 ? launch_gs<4, true, true>(a, ksplit, mode, tiles16, total, stream)
+                : launch_gs<4, false, true>(a, ksplit, mode, tiles16, total, stream);
+    return w1 ? launch_gs<4, true, false>(a, ksplit, mode, tiles16, total, stream)
+              : launch_gs<4, false, false>(a, ksplit, mode, tiles16, total, stream);
   }
   if (w0->bits == 6)
-    return w1 ? launch_gs<6, true, false>(a, ksplit, mode, tiles16, slots, stream)
-              : launch_gs<6, false, false>(a, ksplit, mode, tiles16, slots, stream);
+    return w1 ? launch_gs<6, true, false>(a, ksplit, mode, tiles16, total, stream)
+              : launch_gs<6, false, false>(a, ksplit, mode, tiles16, total, stream);
   if (w0->bits == 2)
-    return w1 ? launch_gs<2, true, false>(a, ksplit, mode, tiles16, slots, stream)
-              : launch_gs<2, false, false>(a, ksplit, mode, tiles16, slots, stream);
+    return w1 ? launch_gs<2, true, false>(a, ksplit, mode, tiles16, total, stream)
+              : launch_gs<2, false, false>(a, ksplit, mode, tiles16, total, stream);
   if (w0->bits == 3)
-    return w1 ? launch_gs<3, true, false>(a, ksplit, mode, tiles16, slots, stream)
-              : launch_gs<3, false, false>(a, ksplit, mode, tiles16, slots, stream);
+    return w1 ? launch_gs<3, true, false>(a, ksplit, mode, tiles16, total, stream)
+              : launch_gs<3, false, false>(a, ksplit, mode, tiles16, total, stream);
   if (w0->bits == 5)
-    return w1 ? launch_gs<5, true, false>(a, ksplit, mode, tiles16, slots, stream)
-              : launch_gs<5, false, false>(a, ksplit, mode, tiles16, slots, stream);
-  return w1 ? launch_gs<8, true, false>(a, ksplit, mode, tiles16, slots, stream)
-            : launch_gs<8, false, false>(a, ksplit, mode, tiles16, slots, stream);
+    return w1 ? launch_gs<5, true, false>(a, ksplit, mode, tiles16, total, stream)
+              : launch_gs<5, false, false>(a, ksplit, mode, tiles16, total, stream);
+  return w1 ? launch_gs<8, true, false>(a, ksplit, mode, tiles16, total, stream)
+            : launch_gs<8, false, false>(a, ksplit, mode, tiles16, total, stream);
 }
 
 

@@ -86,6 +86,17 @@ struct PArgs {
   int hsum_nch, hsum_gs, hsum_G;
   int out_p8;               // GLU: write h in the pair K order (see pair_order)
   int act;                  // GLU: moe_activation of h = act(gate, up)
+  // the shared expert's tiles (expert -1 in the table): its weights, rows and sums
+  struct Shared {
+    const uint16_t* x;
+    const uint16_t* xhl;
+    const uint32_t* w[2];
+    const uint16_t* s[2];
+    const uint16_t* b[2];
+    const uint16_t* lb[2];
+    uint16_t* out;
+    uint16_t* hsum;
+  } sh;
 };
 
 namespace {
@@ -356,7 +367,9 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
   {
     int mat;
     const int wr = code_row(64 * wave + 32 * h + l32, mat);
-    sprow = a.s[mat] + (static_cast<int64_t>(e) * a.N + wr) * G;
+    // (a select of the two arguments: indexed by the lane's matrix, each lane
+    // would first load its pointer from memory)
+    sprow = (mat ? a.s[1] : a.s[0]) + (static_cast<int64_t>(e) * a.N + wr) * G;
   }
   const bool wide = a.wide_scales != 0;
   // chunk j holds groups [c0, c0 + 8), c0 = max(min(8j, G - 8), 0); the
@@ -825,7 +838,8 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
 // for the most tiles P rows can need; the split follows the real counts.  All
 // four bodies share the one LDS allocation (the 128-row body needs the most).
 template <int BITS, bool GLU, bool PAIRS, bool GACT, bool G32>
-__global__ __launch_bounds__(kThreads, 2) void grouped_gemm_prefill_kernel(PArgs a) {
+__global__ __launch_bounds__(kThreads, 2) void grouped_gemm_prefill_kernel(const PArgs args) {
+  PArgs a = args;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[prefill_lds_bytes<BITS, GLU, 4>()];
   const int bid = blockIdx.x;
   const int4 cnt = reinterpret_cast<const int4*>(a.tiles)[0];  // {n4, n3, n2, n1}
@@ -847,7 +861,24 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_prefill_kernel(PArgs
     ntile = v - q * nt;
     slot = nlong + q;
   }
-  const int4 tinfo = reinterpret_cast<const int4*>(a.tiles)[1 + slot];
+  int4 tinfo = reinterpret_cast<const int4*>(a.tiles)[1 + slot];
+  if (tinfo.x < 0) {  // the shared expert: token rows in order
+    tinfo.x = 0;
+    a.x = a.sh.x;
+    a.xhl = a.sh.xhl;
+    a.row_in = nullptr;
+    a.row_out = nullptr;
+    a.gsum_by_pos = 0;
+    a.out = a.sh.out;
+    a.hsum = a.hsum ? a.sh.hsum : nullptr;
+#pragma unroll
+    for (int m = 0; m < 2; ++m) {
+      a.w[m] = a.sh.w[m];
+      a.s[m] = a.sh.s[m];
+      a.b[m] = a.sh.b[m];
+      a.lb[m] = a.sh.lb[m];
+    }
+  }
   if (slot < cnt.x)
     prefill_tile<BITS, GLU, 4, PAIRS, GACT, G32>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
   else if (slot < nlong)
@@ -973,6 +1004,11 @@ bool prefill_supported(const moe_qweight* w0, const moe_qweight* w1) {
   return w0->N % kBN == 0;
 }
 
+bool shared_fits(const moe_qweight& w, const moe_qweight& s) {
+  return s.w && s.experts == 1 && s.N == w.N && s.K == w.K && s.bits == w.bits && s.group_size == w.group_size &&
+         (reinterpret_cast<uintptr_t>(s.w) & 15u) == 0 && (s.biases == nullptr) == (w.biases == nullptr);
+}
+
 // offsets [E+1] on device; tiles: prefill_tile_ints(P, E) ints of scratch
 // (tiles_ready: already built from these offsets);
 // gsum: scratch of max(x_rows, P) * prefill_gsum_stride(w0) 4-byte words.
@@ -1057,10 +1093,32 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
     a.hsum_gs = next_w->group_size;
     a.hsum_G = next_w->K / next_w->group_size;
   }
+  int64_t rows = P, experts = slots;
+  if (pf.shared) {
+    const SharedRows& sh = *pf.shared;
+    if (!sh.w0 || !sh.x || !sh.out || !sh.xhl || (w1 != nullptr) != (sh.w1 != nullptr) || (a.hsum && !sh.hsum) ||
+        !shared_fits(*w0, *sh.w0) || (w1 && !shared_fits(*w1, *sh.w1)))
+      return MOE_E_INVALID_ARG;
+    const moe_qweight* sw[2] = {sh.w0, sh.w1 ? sh.w1 : sh.w0};
+    a.sh.x = sh.x;
+    a.sh.xhl = sh.xhl;
+    a.sh.out = sh.out;
+    a.sh.hsum = sh.hsum;
+    for (int m = 0; m < 2; ++m) {
+      a.sh.w[m] = sw[m]->w;
+      a.sh.s[m] = sw[m]->scales;
+      a.sh.b[m] = sw[m]->biases;
+      a.sh.lb[m] = sw[m]->linear_bias;
+      wide = wide && al16(sw[m]->scales) && (!sw[m]->biases || al16(sw[m]->biases));
+    }
+    a.wide_scales = wide ? 1 : 0;
+    rows += sh.rows;
+    experts += 1;
+  }
   // per XCD: an eighth of the 128- and 96-row tiles, then of the short ones
   // (n4 + n3 <= P/128 + slots, n2 + n1 <= slots: one remainder tile per expert)
   const int64_t nt = a.n_tiles;
-  const int64_t grid = 8 * ((((P / 128 + slots) * nt + 7) / 8) + (2 * slots * nt + 7) / 8);
+  const int64_t grid = 8 * ((((rows / 128 + experts) * nt + 7) / 8) + (2 * experts * nt + 7) / 8);
   if (grid > 0x7fffffffLL) return MOE_E_UNSUPPORTED;
   const unsigned g = static_cast<unsigned>(grid);
   const bool g32 = a.gs == 32;

@@ -299,6 +299,25 @@ def test_block_quantized_shared_gate(T):
     del blk
 
 
+@pytest.mark.parametrize("bits,gs,T", [(4, 64, 1), (4, 64, 2), (4, 64, 63), (8, 32, 33), (6, 64, 17),
+                                       (4, 64, 77), (4, 32, 300), (8, 64, 129), (6, 128, 300)])
+def test_block_shared_in_routed_launches(bits, gs, T):
+    """A shared expert of the routed experts' shape runs in their launches: the per-16-row kernel (few rows
+    per expert, the slots' last one partial) and the large-bucket GEMM (its token tiles in the table, remainders
+    of every height), against the checker."""
+    cfg = W.MoeConfig("shared_small", 60, 1024, 1024, 8, 2, moe.ROUTE_TOPK_PROBS, True, bits, group_size=gs,
+                      shared_intermediate=1024, shared_gated=True)
+    host = W.make_layer(cfg)
+    blk = moe.MoeBlock.from_host(host, DEV)
+    x = W.make_tokens(cfg, T)
+    out, aux = blk.forward(torch.from_numpy(x.view(np.int16)).to(DEV).view(torch.bfloat16), return_aux=True)
+    torch.cuda.synchronize()
+    inds = aux["inds"].cpu().numpy().astype(np.uint32)
+    scores = aux["scores"].cpu().numpy()
+    ref, terms = O.moe_experts(host, x, inds, scores, with_terms=True)
+    assert_close_block(hbf(out), ref, terms, what=f"shared {bits}-bit gs{gs} T={T}", strict_frac=STRICT_FRAC)
+
+
 @pytest.mark.timeout(600)
 @pytest.mark.parametrize("T", [1, 64, 2048])
 def test_block_6bit_experts(T):
