@@ -137,7 +137,7 @@ __device__ void finish_offsets(const int* tot, int64_t P, int E, int* offs_lds, 
   const int c = e < E ? tot[e] : 0;
   int c4 = 0, c3 = 0, c2 = 0, c1 = 0;
   const int ct = e < E ? c : e == E ? o.sh_rows : 0;  // (the shared expert: tiles only; E < NT then)
-  tile_counts(ct, c4, c3, c2, c1);
+  tile_counts(ct, o.half_tiles, c4, c3, c2, c1);
   const int nz = c > 0 ? 1 : 0;
   // rows, 128-row tiles, non-empty | 32-row tiles, 96- | 64-row tiles
   int4 ex = make_int4(c, c4, nz | (c1 << 16), c3 | (c2 << 16)), n;
@@ -165,7 +165,7 @@ __device__ void finish_offsets(const int* tot, int64_t P, int E, int* offs_lds, 
     const int n3 = n.w & 0xffff, n2 = n.w >> 16, n1 = n.z >> 16;
     if (e == 0) reinterpret_cast<int4*>(o.tiles)[0] = make_int4(n.y, n3, n2, n1);
     if (e <= E)
-      write_tiles(o.tiles, e < E ? e : -1, e < E ? ex.x : 0, ct, c4, c3, c2, c1, ex.y, ex.w & 0xffff, ex.w >> 16, ex.z >> 16, n.y, n3, n2);
+      write_tiles(o.tiles, e < E ? e : -1, e < E ? ex.x : 0, ct, o.half_tiles, c4, c3, c2, c1, ex.y, ex.w & 0xffff, ex.w >> 16, ex.z >> 16, n.y, n3, n2);
   }
   __syncthreads();
 }

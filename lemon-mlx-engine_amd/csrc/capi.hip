@@ -578,11 +578,13 @@ int moe_switch_glu(const moe_qweight* gate, const moe_qweight* up, const moe_qwe
   const bool pf_up = moe::use_prefill(P, slots, gate, up), pf_down = moe::use_prefill(P, slots, down, nullptr);
   // the bucketing also writes the large-bucket GEMM's token-tile table (one for both GEMMs)
   p.bk.tiles = pf_up || pf_down ? p.tiles : nullptr;
+  p.bk.half_tiles = pf_up && pf_down && moe::prefill_half_tiles(P, slots, gate, down);
   st = moe::bucket(inds, T, k, E, p.bk, p.bucket_ws, p.bucket_ws_bytes, s);
   if (st != MOE_OK) return st;
   const bool fuse_hsum = pf_up && pf_down;
   moe::PrefillScratch pf1{p.tiles, p.gsum, T, false, fuse_hsum ? p.hsum : nullptr, down};
   pf1.tiles_ready = p.bk.tiles != nullptr;
+  pf1.half_tiles = p.bk.half_tiles;
   pf1.xp = p.xp;
   pf1.act = activation;
   // h in pair K order for a down GEMM that reads it so
@@ -594,6 +596,7 @@ int moe_switch_glu(const moe_qweight* gate, const moe_qweight* up, const moe_qwe
   // down writes each pair's row at its flat index t*k + j: out is [T, k, H]
   moe::PrefillScratch pf2{p.tiles, fuse_hsum ? p.hsum : p.gsum, P, fuse_hsum};
   pf2.tiles_ready = p.bk.tiles != nullptr;
+  pf2.half_tiles = p.bk.half_tiles;
   pf2.in_p8 = h_pairs;
   return moe::grouped_qmm(p.h, nullptr, p.bk.perm, p.bk.offsets, p.bk.active, p.bk.num_active, slots,
                           P, &pf2, down, nullptr, out, s);
@@ -734,6 +737,8 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   // the bucketing also writes the large-bucket GEMM's token-tile table (one for both GEMMs)
   p.bk.tiles = pf_up || pf_down ? p.tiles : nullptr;
   p.bk.sh_rows = sh_large ? static_cast<int>(T) : 0;
+  p.bk.half_tiles = pf_up && pf_down &&
+                    moe::prefill_half_tiles(P + p.bk.sh_rows, slots + (sh_large ? 1 : 0), &d->gate, &d->down);
   // small batches: routing and bucketing in one workgroup, from the partial
   // sums of a router projection spread over many workgroups
   const bool small = moe::route_bucket_small_fits(T, &d->router, p.bk);
@@ -801,6 +806,7 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   pf1.next_gsum = fuse_hsum ? p.hsum : nullptr;
   pf1.next_w = &d->down;
   pf1.tiles_ready = p.bk.tiles != nullptr;
+  pf1.half_tiles = p.bk.half_tiles;
   // (xp_ready false: the large-bucket GEMM writes x in pair order with the group sums)
   pf1.act = d->activation;
   // one token: down and the combine in one launch (h in natural K order)
@@ -861,6 +867,7 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   // so the combine reads a token's k rows without a lookup
   moe::PrefillScratch pf2{p.tiles, fuse_hsum ? p.hsum : p.gsum, P, fuse_hsum};
   pf2.tiles_ready = p.bk.tiles != nullptr;
+  pf2.half_tiles = p.bk.half_tiles;
   pf2.in_p8 = h_pairs;
   if (sh_merged) pf2.shared = &sh2;
   st = moe::grouped_qmm(p.h, nullptr, p.bk.perm, p.bk.offsets, p.bk.active, p.bk.num_active, slots,

@@ -19,7 +19,16 @@ namespace moe {
 // rows); int4 1 + i = tile i {expert, first sorted row, rows, 0}: the n4
 // 128-row tiles (experts in order), then the n3 96-row, the n2 64-row and the
 // n1 32-row tiles.
-__device__ __forceinline__ void tile_counts(int c, int& c4, int& c3, int& c2, int& c1) {
+// half: tiles of at most 64 rows (c / 64 of them, and one of 64 or 32 rows for
+// the remainder), where the tall ones would leave CUs without a workgroup.
+__device__ __forceinline__ void tile_counts(int c, bool half, int& c4, int& c3, int& c2, int& c1) {
+  if (half) {
+    const int r = c & 63;
+    c4 = c3 = 0;
+    c2 = (c >> 6) + (r > 32 ? 1 : 0);
+    c1 = r > 0 && r <= 32 ? 1 : 0;
+    return;
+  }
   const int units = ((c & 127) + 31) >> 5;
   c4 = (c >> 7) + (units == 4 ? 1 : 0);
   c3 = units == 3 ? 1 : 0;
@@ -28,9 +37,14 @@ __device__ __forceinline__ void tile_counts(int c, int& c4, int& c3, int& c2, in
 }
 // Expert e's entries (bucket at sorted row o0, c rows); b4/b3/b2/b1 = its
 // first index within each class, n4/n3/n2 = the class totals.
-__device__ __forceinline__ void write_tiles(int32_t* tiles, int e, int o0, int c, int c4, int c3, int c2, int c1,
-                                            int b4, int b3, int b2, int b1, int n4, int n3, int n2) {
+__device__ __forceinline__ void write_tiles(int32_t* tiles, int e, int o0, int c, bool half, int c4, int c3, int c2,
+                                            int c1, int b4, int b3, int b2, int b1, int n4, int n3, int n2) {
   int4* tab = reinterpret_cast<int4*>(tiles) + 1;
+  if (half) {
+    for (int j = 0; j < c2; ++j) tab[b2 + j] = make_int4(e, o0 + 64 * j, min(64, c - 64 * j), 0);
+    if (c1) tab[n2 + b1] = make_int4(e, o0 + 64 * c2, c - 64 * c2, 0);
+    return;
+  }
   for (int j = 0; j < c4; ++j) tab[b4 + j] = make_int4(e, o0 + 128 * j, min(128, c - 128 * j), 0);
   const int rem0 = o0 + 128 * (c >> 7), r = c & 127;
   if (c3) tab[n4 + b3] = make_int4(e, rem0, r, 0);
@@ -48,6 +62,7 @@ struct BucketOut {
                            //       experts with a non-empty bucket, ascending, then rows = 0
   int32_t* num_active;     // [1]
   int32_t* tiles = nullptr;  // optional: the large-bucket GEMM's token-tile table (prefill_tile_ints)
+  bool half_tiles = false;  // the table's tiles have at most 64 rows (tile_counts)
   int sh_rows = 0;  // > 0: the table also holds the tiles of the shared expert's
                     // sh_rows rows, as one more expert, numbered -1, from row 0
   // the gather_qmm / gather_mm pairs (k = 1): pair i = (b, m), b = i / M, takes
@@ -193,6 +208,7 @@ struct PrefillScratch {
   float* next_gsum = nullptr;
   const moe_qweight* next_w = nullptr;
   bool tiles_ready = false;  // tiles already holds the table for these offsets
+  bool half_tiles = false;   // the table holds tiles of at most 64 rows
   // Pair K order (within 8 consecutive K values: 0, 4, 1, 5, 2, 6, 3, 7): the
   // GEMM reads its operand of 4-bit codes in it at 7 instead of 9 VALU
   // instructions per code word.  gate|up (w1 != NULL) reads its input from
@@ -228,6 +244,9 @@ int grouped_qmm(const uint16_t* x, const int32_t* row_in, const int32_t* row_out
                 int slots, int64_t P, const PrefillScratch* pf, const moe_qweight* w0,
                 const moe_qweight* w1, uint16_t* out, hipStream_t stream);
 bool prefill_supported(const moe_qweight* w0, const moe_qweight* w1);
+// Whether tiles of at most 64 rows suit the large-bucket GEMMs gate|up and down
+// of `rows` rows over at most `experts` non-empty experts.
+bool prefill_half_tiles(int64_t rows, int64_t experts, const moe_qweight* gate, const moe_qweight* down);
 int prefill_gsum_stride(const moe_qweight* w);
 int64_t prefill_tile_ints(int64_t P, int E);
 bool use_prefill(int64_t P, int slots, const moe_qweight* w0, const moe_qweight* w1);

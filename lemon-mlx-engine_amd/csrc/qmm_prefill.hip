@@ -939,7 +939,7 @@ __global__ __launch_bounds__(1024) void make_tiles_kernel(const int32_t* __restr
   __shared__ int base[4][1025];
   const int t = threadIdx.x;
   int c4 = 0, c3 = 0, c2 = 0, c1 = 0;
-  if (t < E) tile_counts(offsets[t + 1] - offsets[t], c4, c3, c2, c1);
+  if (t < E) tile_counts(offsets[t + 1] - offsets[t], false, c4, c3, c2, c1);
   base[0][t] = c4;
   base[1][t] = c3;
   base[2][t] = c2;
@@ -957,7 +957,7 @@ __global__ __launch_bounds__(1024) void make_tiles_kernel(const int32_t* __restr
   }
   __syncthreads();
   if (t < E)
-    write_tiles(tiles, t, offsets[t], offsets[t + 1] - offsets[t], c4, c3, c2, c1, base[0][t], base[1][t], base[2][t],
+    write_tiles(tiles, t, offsets[t], offsets[t + 1] - offsets[t], false, c4, c3, c2, c1, base[0][t], base[1][t], base[2][t],
                 base[3][t], base[0][E], base[1][E], base[2][E]);
 }
 
@@ -983,8 +983,29 @@ int launch_bits(const PArgs& a, bool glu, bool pairs, unsigned grid, hipStream_t
 int prefill_gsum_stride(const moe_qweight* w) { return (w->K / w->group_size + 15) / 16 * 16; }
 
 // header + at most P/128 + E' tiles of 128 rows and E' each of 64 and 32
-// rows, E' = min(E, P) non-empty experts
-int64_t prefill_tile_ints(int64_t P, int E) { return 4 * (1 + P / 128 + 3 * std::min<int64_t>(E, P)); }
+// rows, E' = min(E, P) non-empty experts; of at most 64 rows (prefill_half_tiles:
+// P/128 < kHalfTileWgs then), P/64 + 2 E'
+constexpr int64_t kHalfTileWgs = 512;
+int64_t prefill_tile_ints(int64_t P, int E) {
+  return 4 * (1 + P / 128 + 3 * std::min<int64_t>(E, P) + std::min<int64_t>(P / 128 + 1, kHalfTileWgs));
+}
+
+// Tiles of at most 64 rows where the launch lasts about as long as its longest
+// tile: where the 128-row tiling gives both projections at most two workgroups
+// per CU (one round), and where hardly a bucket holds more than 64 rows.
+// Elsewhere the tall tile's fewer code expansions per row win.  Measured (us,
+// tall | half), workgroups of the wider projection in brackets: SwitchGLU, 1024
+// x 1024, E 32, k 4: T = 256 [320] 75 | 53, 777 [448] 88 | 67, 1024 [512] 91 |
+// 80, 2048 [768] 119 | 129; 2048 x 2048, E 8, k 2: T = 256 [192] 108 | 69, 1024
+// [384] 121 | 105, 2048 [640] 169 | 189; 512 x 1024, E 128, k 8: T = 300 (19 rows
+// per expert) 69 | 57, 500 (31 rows) 74 | 75; Qwen3 block T = 256 (16 rows) 143 |
+// 139, 500 (31 rows) 165 | 167.
+constexpr int kHalfTileRows = 20;  // rows per expert on average
+bool prefill_half_tiles(int64_t rows, int64_t experts, const moe_qweight* gate, const moe_qweight* down) {
+  const int64_t tiles = rows / 128 + experts;
+  return rows < kHalfTileRows * experts ||
+         (tiles * (gate->N / (kBN / 2)) <= kHalfTileWgs && tiles * (down->N / kBN) <= kHalfTileWgs);
+}
 
 bool prefill_supported(const moe_qweight* w0, const moe_qweight* w1) {
   if (w0->bits != 4 && w0->bits != 6 && w0->bits != 8) return false;  // 2, 3, 5 bits: the per-16-row kernel
@@ -1117,8 +1138,11 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
   }
   // per XCD: an eighth of the 128- and 96-row tiles, then of the short ones
   // (n4 + n3 <= P/128 + slots, n2 + n1 <= slots: one remainder tile per expert)
+  // (tiles of at most 64 rows: n2 <= rows/64 + experts, n1 <= experts)
   const int64_t nt = a.n_tiles;
-  const int64_t grid = 8 * ((((rows / 128 + experts) * nt + 7) / 8) + (2 * experts * nt + 7) / 8);
+  const int64_t n_long = pf.half_tiles ? 0 : rows / 128 + experts;
+  const int64_t n_short = 2 * experts + (pf.half_tiles ? rows / 64 : 0);
+  const int64_t grid = 8 * ((n_long * nt + 7) / 8 + (n_short * nt + 7) / 8);
   if (grid > 0x7fffffffLL) return MOE_E_UNSUPPORTED;
   const unsigned g = static_cast<unsigned>(grid);
   const bool g32 = a.gs == 32;

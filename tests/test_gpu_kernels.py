@@ -516,6 +516,15 @@ def test_switch_glu(T, k, E, H, I, bits, gs):
     _switch_glu_case(T, k, E, H, I, bits, gs, False)
 
 
+def test_switch_glu_half_tiles():
+    """Few workgroups: both GEMMs over tiles of at most 64 rows, bucket remainders (mod 64) at both ends of
+    the 32- and 64-row tiles."""
+    counts = [64, 65, 96, 97, 127, 128, 1, 32, 33, 0]
+    inds = np.repeat(np.arange(len(counts), dtype=np.uint32), counts)
+    np.random.default_rng(3).shuffle(inds)
+    _switch_glu_case(inds.size, 1, len(counts), 1024, 1024, 4, 64, False, inds=inds.reshape(-1, 1))
+
+
 @pytest.mark.parametrize("T,k,E,H,I,bits,gs", [(300, 2, 4, 512, 256, 6, 64), (300, 2, 4, 512, 256, 6, 32),
                                                (301, 2, 4, 256, 768, 4, 32), (77, 2, 2, 512, 256, 8, 32)])
 def test_switch_glu_large_buckets_widths(T, k, E, H, I, bits, gs):
@@ -550,7 +559,7 @@ def test_gptoss_swiglu():
     assert_close(hbf(moe.gptoss_swiglu(dbf(a), dbf(b))), h, atol=1e-3, rtol=8e-3)
 
 
-def _switch_glu_case(T, k, E, H, I, bits, gs, biased, act=0):
+def _switch_glu_case(T, k, E, H, I, bits, gs, biased, act=0, inds=None):
     g = W.make_qweight(T + 1, 2, E, I, H, 0.02, gs, bits)
     u = W.make_qweight(T + 1, 3, E, I, H, 0.02, gs, bits)
     d = W.make_qweight(T + 1, 4, E, H, I, 0.02, gs, bits)
@@ -559,7 +568,7 @@ def _switch_glu_case(T, k, E, H, I, bits, gs, biased, act=0):
         for q, tid, sd in ((g, 10, std), (u, 11, std), (d, 12, 0.1)):
             q.linear_bias = W.normal_bf16(T, tid, q.experts * q.N, sd).reshape(q.experts, q.N)
     x = W.normal_bf16(T, 100, T * H, 1.0).reshape(T, H)
-    inds = distinct_inds(T, k, E, seed=T + k)
+    inds = distinct_inds(T, k, E, seed=T + k) if inds is None else inds
     got = hbf(moe.switch_glu(dbf(x), di32(inds), dqw(g), dqw(u), dqw(d), act))
     flat = inds.reshape(-1)
     lhs = np.repeat(np.arange(T, dtype=np.uint32), k)
