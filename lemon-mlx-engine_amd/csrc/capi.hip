@@ -80,13 +80,14 @@ struct BlockPlan {
   int32_t* sh_offsets;
   int32_t* sh_active;
   int32_t* sh_num;
-  int32_t* tiles;
+  int32_t* tiles;      // token-tile table, tall tiles of the routed rows
+  int32_t* tiles_all;  // room for any table (prefill_tile_ints, with the shared expert), or NULL
   int32_t* sh_tiles;
   float* gsum;
   float* hsum;  // group sums of h (written by the gate|up GEMM for down)
   float* rpart;  // small batches: the router projection's partial sums [ks][T][E]
   int rks;       // their slice count (0: the small-batch router is not used)
-  float* sh_hsum;  // group sums of the shared expert's h, as hsum
+  float* sh_hsum;  // group sums of the shared expert's h, as hsum (NULL: no room)
   float* tpart;  // many tokens: the K-split projection's partial sums [tks][T][E]
   int tks;       // their slice count (1: one slice, bf16 logits straight from the projection)
 };
@@ -159,7 +160,15 @@ BlockPlan plan_block(const moe_block_desc* d, int64_t T, void* ws, size_t* total
   p.bk.offsets = c.take<int32_t>(E + 1);
   p.bk.active = c.take<int32_t>(4 * static_cast<int64_t>(E));
   p.bk.num_active = c.take<int32_t>(1);
-  p.tiles = c.take<int32_t>(moe::prefill_tile_ints(P + T, E + 1));  // (with the shared expert's T rows)
+  // the tall tiling of the routed rows; the larger table (64-row tiles, the
+  // shared expert's T rows) takes the logits' place, which the routing has read
+  // before the bucketing writes the table: the workspace, and with it what fits
+  // the static scratch, stays the size of the tall one
+  const int64_t tall_ints = moe::prefill_tall_tile_ints(P, E), all_ints = moe::prefill_tile_ints(P + T, E + 1);
+  p.tiles = c.take<int32_t>(tall_ints);
+  p.tiles_all = all_ints <= tall_ints       ? p.tiles
+                : 2 * all_ints <= T * E     ? reinterpret_cast<int32_t*>(p.logits)
+                                            : nullptr;
   {
     int64_t g = T * moe::prefill_gsum_stride(&d->gate);
     g = std::max<int64_t>(g, P * moe::prefill_gsum_stride(&d->down));
@@ -168,6 +177,12 @@ BlockPlan plan_block(const moe_block_desc* d, int64_t T, void* ws, size_t* total
       g = std::max<int64_t>(g, T * moe::prefill_gsum_stride(&d->shared_down));
     }
     p.gsum = c.take<float>(g);
+    // past the sums of x, where there is room (those of h are in hsum when the
+    // shared expert's are needed)
+    if (d->shared_intermediate > 0) {
+      const int64_t sx = T * moe::prefill_gsum_stride(&d->gate);
+      p.sh_hsum = ws && sx + T * moe::prefill_gsum_stride(&d->shared_down) <= g ? p.gsum + sx : nullptr;
+    }
   }
   p.hsum = c.take<float>(P * moe::prefill_gsum_stride(&d->down));
   p.rks = d->router_q.w ? 0 : moe::router_partial_ks(T, E, H);
@@ -181,7 +196,6 @@ BlockPlan plan_block(const moe_block_desc* d, int64_t T, void* ws, size_t* total
   p.Y = c.take<uint16_t>(P * H);
   if (d->shared_intermediate > 0) {
     p.sgl = c.take<uint16_t>(T);
-    p.sh_hsum = c.take<float>(T * moe::prefill_gsum_stride(&d->shared_down));
     p.hs = c.take<uint16_t>(T * d->shared_intermediate);
     p.Ys = c.take<uint16_t>(T * H);
   }
@@ -189,7 +203,7 @@ BlockPlan plan_block(const moe_block_desc* d, int64_t T, void* ws, size_t* total
     p.sh_offsets = c.take<int32_t>(2);
     p.sh_active = c.take<int32_t>(4);
     p.sh_num = c.take<int32_t>(1);
-    p.sh_tiles = c.take<int32_t>(moe::prefill_tile_ints(T, 1));
+    p.sh_tiles = c.take<int32_t>(moe::prefill_tall_tile_ints(T, 1));
   }
   *total = c.size();
   return p;
@@ -412,7 +426,7 @@ static moe::Carve gqmm_layout(void* ws, int64_t n, int32_t E, int32_t gstride, i
   *active = c.take<int32_t>(4 * static_cast<int64_t>(E));
   *num_active = c.take<int32_t>(1);
   *in_rows = c.take<int32_t>(n);
-  *tiles = c.take<int32_t>(moe::prefill_tile_ints(n, E));
+  *tiles = c.take<int32_t>(moe::prefill_tall_tile_ints(n, E));
   *gsum = c.take<float>(n * gstride);
   *bws_bytes = moe::bucket_workspace_bytes(n, E);
   *bws = c.raw(*bws_bytes);
@@ -475,7 +489,7 @@ static moe::Carve gmm_layout(void* ws, int64_t n, int32_t E, int32_t** perm, int
   *perm = c.take<int32_t>(n);
   *offsets = c.take<int32_t>(E + 1);
   *in_rows = c.take<int32_t>(n);
-  *tiles = c.take<int32_t>(moe::prefill_tile_ints(n, E));
+  *tiles = c.take<int32_t>(moe::prefill_tall_tile_ints(n, E));
   *bws_bytes = moe::bucket_workspace_bytes(n, E);
   *bws = c.raw(*bws_bytes);
   return c;
@@ -719,7 +733,7 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   // rows of one expert: the large-bucket GEMM by itself).
   const bool sh_shape = d->shared_intermediate > 0 && moe::shared_fits(d->gate, d->shared_gate) &&
                         moe::shared_fits(d->up, d->shared_up) && moe::shared_fits(d->down, d->shared_down);
-  const bool sh_large = sh_shape && pf_up && pf_down && E < 1024;
+  const bool sh_large = sh_shape && pf_up && pf_down && E < 1024 && p.tiles_all && p.sh_hsum;
   const bool sh_small = sh_shape && !pf_up && !pf_down && !sh_up_large && !sh_down_large;
   const bool sh_merged = sh_large || sh_small;
   if (rq_large || (!sh_merged && (sh_up_large || sh_down_large))) {
@@ -735,10 +749,11 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   const moe::RouterGroupSums sums{reinterpret_cast<uint16_t*>(p.gsum), d->gate.group_size,
                                   moe::prefill_gsum_stride(&d->gate) / 16};
   // the bucketing also writes the large-bucket GEMM's token-tile table (one for both GEMMs)
-  p.bk.tiles = pf_up || pf_down ? p.tiles : nullptr;
   p.bk.sh_rows = sh_large ? static_cast<int>(T) : 0;
-  p.bk.half_tiles = pf_up && pf_down &&
+  p.bk.half_tiles = pf_up && pf_down && p.tiles_all &&
                     moe::prefill_half_tiles(P + p.bk.sh_rows, slots + (sh_large ? 1 : 0), &d->gate, &d->down);
+  if (sh_large || p.bk.half_tiles) p.tiles = p.tiles_all;
+  p.bk.tiles = pf_up || pf_down ? p.tiles : nullptr;
   // small batches: routing and bucketing in one workgroup, from the partial
   // sums of a router projection spread over many workgroups
   const bool small = moe::route_bucket_small_fits(T, &d->router, p.bk);

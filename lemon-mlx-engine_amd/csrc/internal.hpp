@@ -248,7 +248,8 @@ bool prefill_supported(const moe_qweight* w0, const moe_qweight* w1);
 // of `rows` rows over at most `experts` non-empty experts.
 bool prefill_half_tiles(int64_t rows, int64_t experts, const moe_qweight* gate, const moe_qweight* down);
 int prefill_gsum_stride(const moe_qweight* w);
-int64_t prefill_tile_ints(int64_t P, int E);
+int64_t prefill_tall_tile_ints(int64_t P, int E);  // tiles of up to 128 rows
+int64_t prefill_tile_ints(int64_t P, int E);       // either tiling
 bool use_prefill(int64_t P, int slots, const moe_qweight* w0, const moe_qweight* w1);
 // Whether grouped_qmm's gate|up launch for these arguments can route a single
 // token itself (pf.route): one token (P = k = slots), 4-bit codes with x in

@@ -986,8 +986,9 @@ int prefill_gsum_stride(const moe_qweight* w) { return (w->K / w->group_size + 1
 // rows, E' = min(E, P) non-empty experts; of at most 64 rows (prefill_half_tiles:
 // P/128 < kHalfTileWgs then), P/64 + 2 E'
 constexpr int64_t kHalfTileWgs = 512;
+int64_t prefill_tall_tile_ints(int64_t P, int E) { return 4 * (1 + P / 128 + 3 * std::min<int64_t>(E, P)); }
 int64_t prefill_tile_ints(int64_t P, int E) {
-  return 4 * (1 + P / 128 + 3 * std::min<int64_t>(E, P) + std::min<int64_t>(P / 128 + 1, kHalfTileWgs));
+  return prefill_tall_tile_ints(P, E) + 4 * std::min<int64_t>(P / 128 + 1, kHalfTileWgs);
 }
 
 // Tiles of at most 64 rows where the launch lasts about as long as its longest
