@@ -323,8 +323,7 @@ def test_block_shared_in_routed_launches(bits, gs, T):
 def test_block_6bit_experts(T):
     """Qwen3-30B-A3B shape with 6-bit experts (examples/convert.cpp:10 emits 4/6/8-bit experts;
     examples/test_qbits.cpp:45 runs gather_qmm at 6 bits): every token's routing and output
-    against the checker.  At T = 2048 the buckets (~128 rows) run on the per-16-row kernel,
-    the large-bucket GEMM being 4/8-bit."""
+    against the checker.  At T = 2048 the buckets (~128 rows) run on the large-bucket GEMM."""
     import dataclasses
     _cache.clear()
     gc.collect()
@@ -400,8 +399,8 @@ def test_block_6bit_shared_gate():
 @pytest.mark.parametrize("T", [1500, 2048])
 def test_block_6bit_shared_expert_prefill(T):
     """A 6-bit layer with a sigmoid-gated shared expert at prefill sizes: the shared expert's T rows
-    stay on the per-16-row kernel (the large-bucket GEMM is 4/8-bit), spread over its 64 slots
-    (T = 1500: 32 rows a slot, the last used slot 28; T = 2048: 32 rows in every slot)."""
+    on the per-16-row kernel while the large-bucket GEMM would get fewer than 64 workgroups (gate|up at
+    T = 1500, down at both sizes: 32 rows a slot, at T = 1500 the last used slot 28), else on the GEMM."""
     _cache.clear()
     gc.collect()
     torch.cuda.empty_cache()
