@@ -730,9 +730,12 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   // merged (us): Qwen3-Next T = 1 36.5 | 31.1, 8 77 | 65, 128 199 | 188, 1001
   // 389 | 346; DeepSeek-V3 T = 1 97 | 85, 64 834 | 793, 600 2074 | 1954.  On
   // the per-16-row kernel only while the shared rows would run there too (many
-  // rows of one expert: the large-bucket GEMM by itself).
-  const bool sh_shape = d->shared_intermediate > 0 && moe::shared_fits(d->gate, d->shared_gate) &&
-                        moe::shared_fits(d->up, d->shared_up) && moe::shared_fits(d->down, d->shared_down);
+  // rows of one expert: the large-bucket GEMM by itself).  A launch has one
+  // activation and the shared expert's is always SwiGLU, so routed experts with
+  // another one leave it its own launches.
+  const bool sh_shape = d->shared_intermediate > 0 && d->activation == MOE_ACT_SWIGLU &&
+                        moe::shared_fits(d->gate, d->shared_gate) && moe::shared_fits(d->up, d->shared_up) &&
+                        moe::shared_fits(d->down, d->shared_down);
   const bool sh_large = sh_shape && pf_up && pf_down && E < 1024 && p.tiles_all && p.sh_hsum;
   const bool sh_small = sh_shape && !pf_up && !pf_down && !sh_up_large && !sh_down_large;
   const bool sh_merged = sh_large || sh_small;

@@ -318,6 +318,29 @@ def test_block_shared_in_routed_launches(bits, gs, T):
     assert_close_block(hbf(out), ref, terms, what=f"shared {bits}-bit gs{gs} T={T}", strict_frac=STRICT_FRAC)
 
 
+@pytest.mark.parametrize("act", [moe.ACT_GPTOSS, moe.ACT_GPTOSS_UPSTREAM])
+@pytest.mark.parametrize("T", [1, 17, 300])
+def test_block_shared_expert_keeps_swiglu(T, act):
+    """A shared expert of the routed experts' shape beside routed experts with GPT-OSS's clipped SwiGLU: the
+    shared one always uses SwiGLU (moe_block_desc.activation), at one token, on the per-16-row kernel and on
+    the large-bucket GEMM.  The call without aux (the logits in the workspace) gives the same bytes."""
+    cfg = W.MoeConfig("shared_act", 61, 1024, 1024, 8, 2, moe.ROUTE_TOPK_PROBS, True, 4, shared_intermediate=1024,
+                      shared_gated=True, activation=act)
+    host = W.make_layer(cfg, linear_bias=True)
+    blk = moe.MoeBlock.from_host(host, DEV)
+    x = W.make_tokens(cfg, T)
+    xd = torch.from_numpy(x.view(np.int16)).to(DEV).view(torch.bfloat16)
+    out, aux = blk.forward(xd, return_aux=True)
+    plain = blk.forward(xd)
+    torch.cuda.synchronize()
+    inds = aux["inds"].cpu().numpy().astype(np.uint32)
+    scores = aux["scores"].cpu().numpy()
+    ref, terms = O.moe_experts(host, x, inds, scores, with_terms=True)
+    assert_close_block(hbf(out), ref, terms, what=f"shared expert, activation {act}, T={T}",
+                       strict_frac=STRICT_FRAC, extra=h_rounding_mag(O, host, x, inds, scores))
+    assert (hbf(plain) == hbf(out)).all()
+
+
 @pytest.mark.timeout(600)
 @pytest.mark.parametrize("T", [1, 64, 2048])
 def test_block_6bit_experts(T):
