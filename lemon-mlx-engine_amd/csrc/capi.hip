@@ -739,6 +739,9 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   const bool sh_large = sh_shape && pf_up && pf_down && E < 1024 && p.tiles_all && p.sh_hsum;
   const bool sh_small = sh_shape && !pf_up && !pf_down && !sh_up_large && !sh_down_large;
   const bool sh_merged = sh_large || sh_small;
+  // rows that would not run the large-bucket GEMM by themselves keep the
+  // per-16-row kernel's fp32 group sums in it
+  const bool sh_f32 = sh_large && !(sh_up_large && sh_down_large);
   if (rq_large || (!sh_merged && (sh_up_large || sh_down_large))) {
     MOE_LAUNCH("shared_meta", moe::fill_shared_meta, dim3(1), dim3(64), 0, s, p.sh_offsets, p.sh_active,
                p.sh_num, static_cast<int>(T));
@@ -750,7 +753,8 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   const bool fuse_sums = !qrouter && d->gate.group_size % 64 == 0 && moe::router_tile32(T, d->hidden) &&
                          moe::use_prefill(P, slots, &d->gate, &d->up);
   const moe::RouterGroupSums sums{reinterpret_cast<uint16_t*>(p.gsum), d->gate.group_size,
-                                  moe::prefill_gsum_stride(&d->gate) / 16};
+                                  moe::prefill_gsum_stride(&d->gate) / 16,
+                                  sh_f32 || moe::prefill_f32_sums(&d->gate)};
   // the bucketing also writes the large-bucket GEMM's token-tile table (one for both GEMMs)
   p.bk.sh_rows = sh_large ? static_cast<int>(T) : 0;
   p.bk.half_tiles = pf_up && pf_down && p.tiles_all &&
@@ -827,6 +831,7 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   pf1.half_tiles = p.bk.half_tiles;
   // (xp_ready false: the large-bucket GEMM writes x in pair order with the group sums)
   pf1.act = d->activation;
+  pf1.f32_sums = sh_f32;
   // one token: down and the combine in one launch (h in natural K order)
   const bool dc_fused = T == 1 && !pf_down && moe::down_combine_one_fits(&d->down, k);
   // h in pair K order for a down GEMM that reads it so
@@ -887,6 +892,7 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   pf2.tiles_ready = p.bk.tiles != nullptr;
   pf2.half_tiles = p.bk.half_tiles;
   pf2.in_p8 = h_pairs;
+  pf2.f32_sums = sh_f32;
   if (sh_merged) pf2.shared = &sh2;
   st = moe::grouped_qmm(p.h, nullptr, p.bk.perm, p.bk.offsets, p.bk.active, p.bk.num_active, slots,
                         P, &pf2, &d->down, nullptr, p.Y, s);

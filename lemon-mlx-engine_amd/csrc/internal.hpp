@@ -78,10 +78,11 @@ struct BucketOut {
 
 // Group sums of x produced by the router projection for the expert GEMM
 // (layout of prefill_gsum_stride: nch 16-group chunks of 2 bf16 planes, hi and
-// lo, per row).
+// lo, or with f32 of 16 fp32, per row).
 struct RouterGroupSums {
   uint16_t* xhl;
   int gs, nch;
+  bool f32 = false;
 };
 // Token counts from which the router projection runs the 32x128-tile kernel
 // (the only one that can also emit group sums).
@@ -200,7 +201,7 @@ bool shared_fits(const moe_qweight& w, const moe_qweight& s);
 
 struct PrefillScratch {
   int32_t* tiles;   // [prefill_tile_ints(P, E)] token tile table
-  float* gsum;      // [max(x_rows, P) * prefill_gsum_stride] 4-byte words: group sums as bf16 hi/lo planes
+  float* gsum;      // [max(x_rows, P) * prefill_gsum_stride] 4-byte words: group sums as bf16 hi/lo planes or fp32
   int64_t x_rows;   // rows of x if known, else -1
   bool gsum_ready = false;  // gsum already holds the sums of x's rows (x_rows >= 0)
   // gate|up GEMM only: also write the group sums of its output rows (h), for
@@ -233,6 +234,9 @@ struct PrefillScratch {
   // the shared expert in the same launch (the token-tile table then holds its
   // tiles: BucketOut::sh_rows)
   const SharedRows* shared = nullptr;
+  // large-bucket GEMM: fp32 group sums (gsum, and next_gsum where written here)
+  // also where the weights do not ask for them (prefill_f32_sums)
+  bool f32_sums = false;
 };
 constexpr int kOneExpertSlots = 64;
 inline int one_expert_slots(int64_t P) { return static_cast<int>(std::min<int64_t>((P + 15) / 16, kOneExpertSlots)); }
@@ -248,6 +252,9 @@ bool prefill_supported(const moe_qweight* w0, const moe_qweight* w1);
 // of `rows` rows over at most `experts` non-empty experts.
 bool prefill_half_tiles(int64_t rows, int64_t experts, const moe_qweight* gate, const moe_qweight* down);
 int prefill_gsum_stride(const moe_qweight* w);
+// Whether the large-bucket GEMM keeps the group sums of w's input rows in fp32
+// (else as two bf16 parts).
+bool prefill_f32_sums(const moe_qweight* w);
 int64_t prefill_tall_tile_ints(int64_t P, int E);  // tiles of up to 128 rows
 int64_t prefill_tile_ints(int64_t P, int E);       // either tiling
 bool use_prefill(int64_t P, int slots, const moe_qweight* w0, const moe_qweight* w1);

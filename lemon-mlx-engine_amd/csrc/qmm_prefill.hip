@@ -18,7 +18,17 @@
 // the groups run on the MFMA while the K pipeline fills, written as
 // X.b + (-OFF X).s so that its weight-side operands are the checkpoint's own
 // bf16 biases and scales; X is split into bf16 hi + lo parts (exact to 2^-16
-// relative) and -OFF X is exact.
+// relative) and -OFF X is exact.  F32S instantiations (prefill_f32_sums: 6-bit
+// codes and groups of 32; a launch that also takes the rows of a shared expert
+// too small for this GEMM by itself) keep X whole: it is stored in fp32, in the
+// two parts' room, and split into three bf16 parts (24 bits) in registers, and
+// SiLU divides instead of taking v_rcp_f32 -- the precision of the per-16-row
+// kernel, where those rows run at other sizes.  Relative error against 64 bits
+// (2-norm), two parts | three: SwitchGLU 1024 x 1024, groups of 32, T = 777
+// 0.0041313 | 0.0041264; one projection of groups of 32 at 4 bits, 2048 x 768, T = 500
+// 0.0016633 | 0.0016625; the per-16-row kernel 0.0041260 and 0.0016625.  Whole calls
+// (us): Qwen3 block of 6 bits, T = 2048, 371 | 376, Qwen3-Next block T = 1001
+// 343 | 344, the SwitchGLU above 72.7 | 72.5.
 //
 // Tiling.  A workgroup of 4 waves computes a BM x 256 tile of one expert:
 // BM = 32*MT token rows by 256 weight rows (GLU: 128 gate rows and the 128
@@ -68,6 +78,7 @@ struct PArgs {
   const int32_t* row_in;    // sorted pos -> input row (NULL: pos)
   const int32_t* row_out;   // sorted pos -> output row (NULL: pos)
   const uint16_t* xhl;      // [*, nch, 32] group sums X of the input rows: bf16 hi(16) | lo(16) per chunk
+                            // (F32S: 16 fp32 in the chunk's 64 bytes)
   int nch;                  // 16-group chunks per row (G rounded up to 16, / 16)
   int gsum_by_pos;          // xhl rows: 1 = sorted position, 0 = input row (as x)
   const int32_t* tiles;     // [0] = token tile count; entry i at 4+4i: {expert, row0, rows, 0}
@@ -84,6 +95,7 @@ struct PArgs {
   // projection, in the xhl layout (nch chunks of 2 bf16 planes), groups of gs
   uint16_t* hsum;
   int hsum_nch, hsum_gs, hsum_G;
+  int hsum_f32;             // the sums of h as fp32 (the next projection's launch is F32S)
   int out_p8;               // GLU: write h in the pair K order (see pair_order)
   int act;                  // GLU: moe_activation of h = act(gate, up)
   // the shared expert's tiles (expert -1 in the table): its weights, rows and sums
@@ -122,6 +134,9 @@ constexpr int kChunkBytesOf = 64 * kChunkRowOf<BITS>;  // one wave's 64 rows of 
 // kernel's, and its last bit changes the bf16 h in a few outputs only)
 __device__ __forceinline__ float silu(float g) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)); }
 
+// the same with a correctly rounded division (F32S)
+__device__ __forceinline__ float silu_div(float g) { return g / (1.0f + __expf(-g)); }
+
 // hi = bf16(v) (round to nearest even), lo = bf16(v - hi); v - hi is exact in fp32.
 __device__ __forceinline__ void split_bf16(float v, uint16_t& hi, uint16_t& lo) {
   hi = f2bf(v);
@@ -140,6 +155,23 @@ __device__ __forceinline__ uint32_t and_or(uint32_t v, uint32_t m, uint32_t c) {
   uint32_t r;
   asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "s"(m), "v"(c));
   return r;
+}
+
+// eight fp32 -> three bf16 operands whose sum is the value: hi = bf16(v), the
+// residual of 16 bits as mid + lo (each subtraction exact; an infinite v has
+// residual 0)
+__device__ __forceinline__ void split3_bf16(const u32x4 (&v)[2], u32x4& hi, u32x4& mid, u32x4& lo) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float a = __uint_as_float(v[q >> 1][2 * (q & 1)]), b = __uint_as_float(v[q >> 1][2 * (q & 1) + 1]);
+    const uint32_t h = pk_bf16(a, b);
+    const float ha = __uint_as_float(h << 16), hb = __uint_as_float(h & 0xffff0000u);
+    const float ra = __builtin_isinf(ha) ? 0.0f : a - ha, rb = __builtin_isinf(hb) ? 0.0f : b - hb;
+    const uint32_t m = pk_bf16(ra, rb);
+    hi[q] = h;
+    mid[q] = m;
+    lo[q] = pk_bf16(ra - __uint_as_float(m << 16), rb - __uint_as_float(m & 0xffff0000u));
+  }
 }
 
 // Pair K order (pair_pos, to_pair_order): the GEMM reads a stored 16-byte
@@ -246,7 +278,8 @@ constexpr int prefill_lds_bytes() {
 // compiled (the selector's other branches, inlined into every tile height's
 // unrolled epilogue, doubled the kernel's code and cost ~4 % of gate|up).
 // G32: groups of 32, two per K step (another K order, below, and two folds).
-template <int BITS, bool GLU, int MT, bool PAIRS, bool GACT, bool G32>
+// F32S: whole fp32 group sums and a dividing SiLU (file header).
+template <int BITS, bool GLU, int MT, bool PAIRS, bool GACT, bool G32, bool F32S>
 __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const int e, const int row0,
                                              const int rows, const int ntile) {
   constexpr int BM = 32 * MT;
@@ -507,22 +540,33 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
       // one m-tile's group sums at a time (few registers live beside acc)
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        u32x4 xv[2];  // hi, lo of groups 16c + 8h .. +7 of row m
+        constexpr int kParts = F32S ? 3 : 2;
+        u32x4 xv[kParts];  // hi, lo (F32S: hi, mid, lo) of groups 16c + 8h .. +7 of row m
         const int m = mt * 32 + l32;
+        if constexpr (F32S) {
+          u32x4 f[2];
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
-          xv[q] = *reinterpret_cast<const u32x4*>(zs + m * 128 + 16 * ((4 * (c & 1) + 2 * q + h) ^ ((m >> 1) & 7)));
+          for (int q = 0; q < 2; ++q)
+            f[q] = *reinterpret_cast<const u32x4*>(zs + m * 128 + 16 * ((4 * (c & 1) + 2 * h + q) ^ ((m >> 1) & 7)));
+          split3_bf16(f, xv[0], xv[1], xv[2]);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+            xv[q] = *reinterpret_cast<const u32x4*>(zs + m * 128 + 16 * ((4 * (c & 1) + 2 * q + h) ^ ((m >> 1) & 7)));
+        }
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
           const bf16x8 bB = __builtin_bit_cast(bf16x8, bw[nt]);
           const bf16x8 sB = __builtin_bit_cast(bf16x8, sw[nt]);
           if (has_b) {
-            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xv[0]), bB, acc[mt][nt], 0, 0, 0);
-            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xv[1]), bB, acc[mt][nt], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < kParts; ++q)
+              acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xv[q]), bB, acc[mt][nt], 0, 0, 0);
           }
           if constexpr (OFF != 0) {
-            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xv[0]), sB, acc[mt][nt], 0, 0, 0);
-            acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xv[1]), sB, acc[mt][nt], 0, 0, 0);
+#pragma unroll
+            for (int q = 0; q < kParts; ++q)
+              acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, xv[q]), sB, acc[mt][nt], 0, 0, 0);
           }
         }
         // keep the next m-tile's loads below this point (register pressure)
@@ -759,8 +803,9 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
           u1 = bfr(u1 + lbv[1]);
         }
         uint32_t hv;
-        if constexpr (GACT) hv = pk_bf16(glu_act(a.act, g0, u0, silu(g0)), glu_act(a.act, g1, u1, silu(g1)));
-        else hv = pk_bf16(silu(g0) * u0, silu(g1) * u1);
+        const float s0 = F32S ? silu_div(g0) : silu(g0), s1 = F32S ? silu_div(g1) : silu(g1);
+        if constexpr (GACT) hv = pk_bf16(glu_act(a.act, g0, u0, s0), glu_act(a.act, g1, u1, s1));
+        else hv = pk_bf16(s0 * u0, s1 * u1);
         ot[m0 * OS + hcol] = static_cast<uint16_t>(hv);
         ot[(m0 + 1) * OS + hcol] = static_cast<uint16_t>(hv >> 16);
       } else {
@@ -814,16 +859,22 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
         }
         uint16_t* dst = a.hsum + static_cast<int64_t>(hs_row[i]) * a.hsum_nch * 32;
         const int g = ntile * gpt + q;
-        uint16_t hi, lo;
-        split_bf16(sum, hi, lo);
-        uint16_t* c = dst + (g >> 4) * 32 + (g & 15);
-        c[0] = hi;
-        c[16] = lo;
         // groups past the last one are zero (written by the first column tile)
-        if (ntile == 0 && q == 0)
-          for (int gz = a.hsum_G; gz < 16 * a.hsum_nch; ++gz)
+        const int g_end = ntile == 0 && q == 0 ? 16 * a.hsum_nch : 0;
+        if (a.hsum_f32) {
+          float* dst32 = reinterpret_cast<float*>(dst);
+          dst32[g] = sum;
+          for (int gz = a.hsum_G; gz < g_end; ++gz) dst32[gz] = 0.0f;
+        } else {
+          uint16_t hi, lo;
+          split_bf16(sum, hi, lo);
+          uint16_t* c = dst + (g >> 4) * 32 + (g & 15);
+          c[0] = hi;
+          c[16] = lo;
+          for (int gz = a.hsum_G; gz < g_end; ++gz)
 #pragma unroll
             for (int pl = 0; pl < 2; ++pl) dst[(gz >> 4) * 32 + 16 * pl + (gz & 15)] = 0;
+        }
       }
     }
   }
@@ -837,7 +888,7 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
 // robin, so that the last workgroups to run are short ones.  The grid is sized
 // for the most tiles P rows can need; the split follows the real counts.  All
 // four bodies share the one LDS allocation (the 128-row body needs the most).
-template <int BITS, bool GLU, bool PAIRS, bool GACT, bool G32>
+template <int BITS, bool GLU, bool PAIRS, bool GACT, bool G32, bool F32S>
 __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_prefill_kernel(const PArgs args) {
   PArgs a = args;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[prefill_lds_bytes<BITS, GLU, 4>()];
@@ -880,25 +931,25 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_prefill_kernel(const
     }
   }
   if (slot < cnt.x)
-    prefill_tile<BITS, GLU, 4, PAIRS, GACT, G32>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+    prefill_tile<BITS, GLU, 4, PAIRS, GACT, G32, F32S>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
   else if (slot < nlong)
-    prefill_tile<BITS, GLU, 3, PAIRS, GACT, G32>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+    prefill_tile<BITS, GLU, 3, PAIRS, GACT, G32, F32S>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
   else if (slot < nlong + cnt.z)
-    prefill_tile<BITS, GLU, 2, PAIRS, GACT, G32>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+    prefill_tile<BITS, GLU, 2, PAIRS, GACT, G32, F32S>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
   else
-    prefill_tile<BITS, GLU, 1, PAIRS, GACT, G32>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+    prefill_tile<BITS, GLU, 1, PAIRS, GACT, G32, F32S>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
 }
 
 // xhl[r] = the group sums X[g] (fp32) of row src(r) as bf16 hi and lo parts,
 // (xp != NULL: also row r of x in pair K order, xp[r] = pairs(x[r]));
-// in 16-group chunks [hi(16) | lo(16)]; groups past G are zero.
+// in 16-group chunks [hi(16) | lo(16)] (f32: 16 fp32); groups past G are zero.
 // src(r) = row_in ? row_in[r] : r.  L = gs/8 consecutive lanes own one group
 // (16 bytes each: whole 128-byte lines per 8 lanes) and add their partial
 // sums across the DPP row; groups are numbered over rows x 16*nch.
 template <int L>
 __global__ __launch_bounds__(256) void group_sums_kernel(const uint16_t* __restrict__ x,
                                                          const int32_t* __restrict__ row_in, int64_t R, int K,
-                                                         int nch, uint16_t* __restrict__ xhl,
+                                                         int nch, int f32, uint16_t* __restrict__ xhl,
                                                          uint16_t* __restrict__ xp) {
   const int64_t tid = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   const int part = threadIdx.x & (L - 1);
@@ -925,6 +976,10 @@ __global__ __launch_bounds__(256) void group_sums_kernel(const uint16_t* __restr
   if constexpr (L >= 8) s += dpp_f<kDppHalfMirror>(s);
   if constexpr (L == 16) s += dpp_f<kDppMirror>(s);
   if (part == 0 && r < R) {
+    if (f32) {
+      reinterpret_cast<float*>(xhl)[r * nch * 16 + g] = s;
+      return;
+    }
     uint16_t hi, lo;
     split_bf16(s, hi, lo);
     uint16_t* c = xhl + r * nch * 32 + (g >> 4) * 32 + (g & 15);
@@ -961,25 +1016,35 @@ __global__ __launch_bounds__(1024) void make_tiles_kernel(const int32_t* __restr
                 base[3][t], base[0][E], base[1][E], base[2][E]);
 }
 
-template <int BITS, bool GLU, bool PAIRS, bool GACT, bool G32>
+template <int BITS, bool GLU, bool PAIRS, bool GACT, bool G32, bool F32S>
 int launch_prefill(const PArgs& a, unsigned grid, hipStream_t stream) {
-  MOE_LAUNCH(GLU ? "gemm_gate_up_swiglu" : "gemm_down", (grouped_gemm_prefill_kernel<BITS, GLU, PAIRS, GACT, G32>),
-             dim3(grid), dim3(kThreads), 0, stream, a);
+  MOE_LAUNCH(GLU ? "gemm_gate_up_swiglu" : "gemm_down",
+             (grouped_gemm_prefill_kernel<BITS, GLU, PAIRS, GACT, G32, F32S>), dim3(grid), dim3(kThreads), 0, stream, a);
   return launch_status("grouped_gemm_prefill");
 }
 
 template <int BITS, bool G32>
-int launch_bits(const PArgs& a, bool glu, bool pairs, unsigned grid, hipStream_t stream) {
+int launch_bits(const PArgs& a, bool glu, bool pairs, bool f32, unsigned grid, hipStream_t stream) {
+  constexpr bool kF32 = BITS == 6 || G32;  // (prefill_f32_sums)
+  if constexpr (!kF32) {
+    // with the shared expert's rows: SwiGLU, and h in pair order
+    if (f32 && ((glu && a.act != MOE_ACT_SWIGLU) || (!glu && !pairs))) return MOE_E_INVALID_ARG;
+    if (f32)
+      return glu ? launch_prefill<BITS, true, true, false, G32, true>(a, grid, stream)
+                 : launch_prefill<BITS, false, true, false, G32, true>(a, grid, stream);
+  }
   if (glu)
-    return a.act != MOE_ACT_SWIGLU ? launch_prefill<BITS, true, true, true, G32>(a, grid, stream)
-                                   : launch_prefill<BITS, true, true, false, G32>(a, grid, stream);
-  return pairs ? launch_prefill<BITS, false, true, false, G32>(a, grid, stream)
-               : launch_prefill<BITS, false, false, false, G32>(a, grid, stream);
+    return a.act != MOE_ACT_SWIGLU ? launch_prefill<BITS, true, true, true, G32, kF32>(a, grid, stream)
+                                   : launch_prefill<BITS, true, true, false, G32, kF32>(a, grid, stream);
+  return pairs ? launch_prefill<BITS, false, true, false, G32, kF32>(a, grid, stream)
+               : launch_prefill<BITS, false, false, false, G32, kF32>(a, grid, stream);
 }
 
 }  // namespace
 
-// 4-byte words per row of the group-sum buffer: 32 bf16 per 16-group chunk
+bool prefill_f32_sums(const moe_qweight* w) { return w->bits == 6 || w->group_size == 32; }
+
+// 4-byte words per row of the group-sum buffer: 32 bf16 or 16 fp32 per 16-group chunk
 int prefill_gsum_stride(const moe_qweight* w) { return (w->K / w->group_size + 15) / 16 * 16; }
 
 // header + at most P/128 + E' tiles of 128 rows and E' each of 64 and 32
@@ -1052,6 +1117,7 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
   // the kernel addresses x with 32-bit byte offsets
   if ((x_rows >= 0 ? x_rows : P) * static_cast<int64_t>(w0->K) * 2 >= (int64_t{1} << 32)) return MOE_E_UNSUPPORTED;
   const int gstride = prefill_gsum_stride(w0);
+  const bool f32 = pf.f32_sums || prefill_f32_sums(w0);
   const bool by_pos = x_rows < 0;
   const int64_t R = by_pos ? P : x_rows;
   if (R > 0 && !(pf.gsum_ready && !by_pos)) {
@@ -1063,13 +1129,13 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
     const int32_t* rin = by_pos ? row_in : nullptr;
     if (L == 4)
       MOE_LAUNCH("group_sums", group_sums_kernel<4>, grid, dim3(256), 0, stream, x, rin, R, w0->K, gstride / 16,
-                 reinterpret_cast<uint16_t*>(gsum), xp);
+                 f32, reinterpret_cast<uint16_t*>(gsum), xp);
     else if (L == 8)
       MOE_LAUNCH("group_sums", group_sums_kernel<8>, grid, dim3(256), 0, stream, x, rin, R, w0->K, gstride / 16,
-                 reinterpret_cast<uint16_t*>(gsum), xp);
+                 f32, reinterpret_cast<uint16_t*>(gsum), xp);
     else
       MOE_LAUNCH("group_sums", group_sums_kernel<16>, grid, dim3(256), 0, stream, x, rin, R, w0->K, gstride / 16,
-                 reinterpret_cast<uint16_t*>(gsum), xp);
+                 f32, reinterpret_cast<uint16_t*>(gsum), xp);
     MOE_CHECK_LAUNCH("group_sums");
   }
   if (!pf.tiles_ready) {
@@ -1114,6 +1180,7 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
     a.hsum_nch = prefill_gsum_stride(next_w) / 16;
     a.hsum_gs = next_w->group_size;
     a.hsum_G = next_w->K / next_w->group_size;
+    a.hsum_f32 = pf.f32_sums || prefill_f32_sums(next_w) ? 1 : 0;
   }
   int64_t rows = P, experts = slots;
   if (pf.shared) {
@@ -1148,10 +1215,13 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
   const unsigned g = static_cast<unsigned>(grid);
   const bool g32 = a.gs == 32;
   if (w0->bits == 4)
-    return g32 ? launch_bits<4, true>(a, w1, pf.in_p8, g, stream) : launch_bits<4, false>(a, w1, pf.in_p8, g, stream);
+    return g32 ? launch_bits<4, true>(a, w1, pf.in_p8, f32, g, stream)
+               : launch_bits<4, false>(a, w1, pf.in_p8, f32, g, stream);
   if (w0->bits == 6)
-    return g32 ? launch_bits<6, true>(a, w1, pf.in_p8, g, stream) : launch_bits<6, false>(a, w1, pf.in_p8, g, stream);
-  return g32 ? launch_bits<8, true>(a, w1, pf.in_p8, g, stream) : launch_bits<8, false>(a, w1, pf.in_p8, g, stream);
+    return g32 ? launch_bits<6, true>(a, w1, pf.in_p8, f32, g, stream)
+               : launch_bits<6, false>(a, w1, pf.in_p8, f32, g, stream);
+  return g32 ? launch_bits<8, true>(a, w1, pf.in_p8, f32, g, stream)
+             : launch_bits<8, false>(a, w1, pf.in_p8, f32, g, stream);
 }
 
 }  // namespace moe

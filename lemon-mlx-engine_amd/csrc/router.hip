@@ -258,9 +258,9 @@ struct RouterGemmArgs {
   const uint16_t* bias;  // [E] or NULL, added before the one rounding
   uint16_t* out;
   int T, E, H;
-  // group sums (xhl != nullptr): xhl[t] in 16-group chunks [hi(16) | lo(16)],
-  // groups of gs along H, groups G..16*nch-1 zero (the layout the expert GEMM
-  // reads)
+  // group sums (xhl != nullptr): xhl[t] in 16-group chunks [hi(16) | lo(16)]
+  // (f32: 16 fp32), groups of gs along H, groups G..16*nch-1 zero (the layout
+  // the expert GEMM reads)
   uint16_t* xhl;
   int gs, nch;
   // optional: x in pair K order, written from the staged token rows by the
@@ -269,6 +269,7 @@ struct RouterGemmArgs {
   // K split over gridDim.z workgroups (> 1): fp32 partial sums [KS][T][E]
   // (no bias) instead of out; workgroup ks takes K steps [ks S, (ks+1) S)
   float* part;
+  int f32;
 };
 
 constexpr int kRStages = 4;
@@ -359,10 +360,15 @@ __global__ __launch_bounds__(256) void router_gemm_tile32(RouterGemmArgs a) {
           if ((gi & 7) == 7 || s == S - 1) {
             const int g = (gi & ~7) + cu;  // groups of this slice only: [s0 / spg, gi]
             if (m0 + crow < a.T && g <= gi && g >= s0 / spg) {
-              const uint16_t hi = f2bf(gmine), lo = f2bf(gmine - bf2f(hi));
-              uint16_t* c = a.xhl + static_cast<int64_t>(m0 + crow) * a.nch * 32 + (g >> 4) * 32 + (g & 15);
-              c[0] = hi;
-              c[16] = lo;
+              uint16_t* row = a.xhl + static_cast<int64_t>(m0 + crow) * a.nch * 32;
+              if (a.f32) {
+                reinterpret_cast<float*>(row)[g] = gmine;
+              } else {
+                const uint16_t hi = f2bf(gmine), lo = f2bf(gmine - bf2f(hi));
+                uint16_t* c = row + (g >> 4) * 32 + (g & 15);
+                c[0] = hi;
+                c[16] = lo;
+              }
             }
           }
         }
@@ -402,9 +408,14 @@ __global__ __launch_bounds__(256) void router_gemm_tile32(RouterGemmArgs a) {
   }
   if (sums && wave == 0 && ks == 0 && h == 0 && m0 + r < a.T) {
     uint16_t* row = a.xhl + static_cast<int64_t>(m0 + r) * a.nch * 32;
-    for (int gi = a.H / a.gs; gi < 16 * a.nch; ++gi)
+    for (int gi = a.H / a.gs; gi < 16 * a.nch; ++gi) {
+      if (a.f32) {
+        reinterpret_cast<float*>(row)[gi] = 0.0f;
+        continue;
+      }
 #pragma unroll
       for (int q = 0; q < 2; ++q) row[(gi >> 4) * 32 + 16 * q + (gi & 15)] = 0;
+    }
   }
 }
 
@@ -552,12 +563,13 @@ int router_logits(const uint16_t* x, const uint16_t* wg, const uint16_t* bias, i
     MOE_LAUNCH("router_logits", row_dot_kernel, dim3(static_cast<unsigned>((T + 3) / 4)), dim3(256), 0, stream, x, wg,
                bias, T, H, logits);
   } else if (router_tile32(T, H)) {
-    RouterGemmArgs a{x, wg, bias, logits, static_cast<int>(T), E, H, nullptr, 64, 0, xp, nullptr};
+    RouterGemmArgs a{x, wg, bias, logits, static_cast<int>(T), E, H, nullptr, 64, 0, xp, nullptr, 0};
     if (sums) {
       if (sums->gs % 64 != 0 || H % sums->gs != 0 || sums->nch * 16 < H / sums->gs) return MOE_E_INVALID_ARG;
       a.xhl = sums->xhl;
       a.gs = sums->gs;
       a.nch = sums->nch;
+      a.f32 = sums->f32;
     }
     dim3 grid(static_cast<unsigned>((T + 31) / 32), (E + 127) / 128);
     MOE_LAUNCH("router_logits", router_gemm_tile32, grid, dim3(256), 0, stream, a);
@@ -593,13 +605,14 @@ int router_partials_tile32(const uint16_t* x, const uint16_t* wg, int64_t T, int
   if (!x || !wg || !part || ks < 2 || T < 1 || E <= 0 || !router_tile32(T, H)) return MOE_E_INVALID_ARG;
   if (!aligned16(x) || !aligned16(wg) || (xp && !aligned16(xp))) return MOE_E_UNSUPPORTED;
   if (T > 0x7fffffffLL - 32 || (H / 64) % ks != 0) return MOE_E_UNSUPPORTED;
-  RouterGemmArgs a{x, wg, nullptr, nullptr, static_cast<int>(T), E, H, nullptr, 64, 0, xp, part};
+  RouterGemmArgs a{x, wg, nullptr, nullptr, static_cast<int>(T), E, H, nullptr, 64, 0, xp, part, 0};
   if (sums) {
     if (sums->gs % 64 != 0 || H % sums->gs != 0 || sums->nch * 16 < H / sums->gs) return MOE_E_INVALID_ARG;
     if ((H / 64 / ks) % (sums->gs / 64) != 0) return MOE_E_UNSUPPORTED;  // each slice holds whole groups
     a.xhl = sums->xhl;
     a.gs = sums->gs;
     a.nch = sums->nch;
+    a.f32 = sums->f32;
   }
   dim3 grid(static_cast<unsigned>((T + 31) / 32), (E + 127) / 128, ks);
   MOE_LAUNCH("router_logits", router_gemm_tile32, grid, dim3(256), 0, stream, a);

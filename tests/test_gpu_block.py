@@ -318,6 +318,37 @@ def test_block_shared_in_routed_launches(bits, gs, T):
     assert_close_block(hbf(out), ref, terms, what=f"shared {bits}-bit gs{gs} T={T}", strict_frac=STRICT_FRAC)
 
 
+@pytest.mark.parametrize("bits,T", [(4, 300), (8, 300), (4, 600)])
+def test_block_shared_whole_group_sums(bits, T):
+    """A shared expert of the routed shape in the large-bucket launches, too few rows for the GEMM by itself:
+    its group sums keep fp32 there (T = 600: those the router projection writes).  Sums of 2^17 + 2^8 + 1 against
+    gate and up weights that are 0 as -q + 8 at q = 8, and 1 in the last column, where x is 1: gate and up are
+    exactly 1 (off by 8 or 136 if the sums lose their last bit); every partial sum is exact in fp32 (multiples of
+    8 until the last group).  Routed experts of zeros."""
+    cfg = W.MoeConfig("shared_sums", 62, 1024, 1024, 8, 2, moe.ROUTE_TOPK_PROBS, True, bits, shared_intermediate=1024)
+    host = W.make_layer(cfg)
+    host.router_weight[:] = 0
+    for q in (host.gate, host.up, host.down):
+        q.scales[:] = 0
+        q.biases[:] = 0
+    per = 32 // bits
+    for q in host.shared[:2]:
+        q.scales[:] = to_bf16(np.float32(-1.0))
+        q.biases[:] = to_bf16(np.float32(8.0))
+        q.w[:] = sum(8 << (bits * i) for i in range(per))
+        q.w[:, :, -1] -= np.uint32(1 << (32 - bits))  # the last column: code 7
+    x = np.zeros((T, cfg.hidden), np.float32)
+    x[:, -1] = 1.0
+    for t in range(T):
+        x[t, 64 * (t % 15) + np.array([3, 29, 62])] = [2.0 ** 17, 2.0 ** 8, 1.0]
+    x = to_bf16(x)
+    blk = moe.MoeBlock.from_host(host, DEV)
+    out, aux = blk.forward(torch.from_numpy(x.view(np.int16)).to(DEV).view(torch.bfloat16), return_aux=True)
+    torch.cuda.synchronize()
+    ref = O.moe_experts(host, x, aux["inds"].cpu().numpy().astype(np.uint32), aux["scores"].cpu().numpy())
+    assert_close(hbf(out), ref, what="shared expert, whole group sums")
+
+
 @pytest.mark.parametrize("act", [moe.ACT_GPTOSS, moe.ACT_GPTOSS_UPSTREAM])
 @pytest.mark.parametrize("T", [1, 17, 300])
 def test_block_shared_expert_keeps_swiglu(T, act):

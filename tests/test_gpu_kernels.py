@@ -329,6 +329,30 @@ def test_gather_qmm_tile_classes_widths(bits, gs, K):
     _tile_classes_case(bits, gs, K)
 
 
+@pytest.mark.parametrize("bits,gs", [(6, 64), (6, 128), (6, 32), (4, 32), (8, 32)])
+def test_gather_qmm_whole_group_sums(bits, gs):
+    """Group sums of 18 bits (2^17 + 2^8 + 1) against weights that are 0 as s q + b = -s' q + 8 s' at q = 8
+    (s' a power of two): every product and sum is exact in fp32, so the output is exactly 0 if the group sums
+    keep fp32, and 8 s' or 136 s' if their last bit is lost."""
+    E, N, K, batch = 4, 2048, 512, 80
+    G = K // gs
+    stream = int.from_bytes(np.full(32, 0, np.uint8).tobytes(), "little")
+    for i in range(32):
+        stream |= 8 << (bits * i)
+    words = np.frombuffer(stream.to_bytes(4 * bits, "little"), np.uint32)
+    scale = 2.0 ** (np.arange(G) % 3)
+    q = W.HostQWeight(np.tile(words, (E, N, K // 32)).astype(np.uint32),
+                      np.broadcast_to(to_bf16(-scale), (E, N, G)).copy(),
+                      np.broadcast_to(to_bf16(8 * scale), (E, N, G)).copy(), E, N, K, gs, bits)
+    x = np.zeros((batch, K), np.float32)
+    rng = np.random.default_rng(bits + gs)
+    for r in range(batch):
+        x[r, gs * (r % G) + rng.choice(gs, 3, replace=False)] = [2.0 ** 17, 2.0 ** 8, 1.0]
+    rhs = rng.integers(0, E, batch).astype(np.uint32)
+    got = moe.gather_qmm(dbf(to_bf16(x)), dqw(q), None, di32(rhs))
+    assert (got == 0).all()
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 def test_gather_qmm_tile_classes(bits):
     """Bucket remainders (mod 128 rows) of 0, 1, 32, 33, 64, 65, 96, 97 and 127
