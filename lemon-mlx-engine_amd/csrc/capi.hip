@@ -589,7 +589,7 @@ int moe_switch_glu(const moe_qweight* gate, const moe_qweight* up, const moe_qwe
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int E = gate->experts;
   const int slots = static_cast<int>(P < E ? P : E);
-  const bool pf_up = moe::use_prefill(P, slots, gate, up), pf_down = moe::use_prefill(P, slots, down, nullptr);
+  const bool pf_up = moe::use_prefill(P, slots, gate, up, T), pf_down = moe::use_prefill(P, slots, down, nullptr);
   // the bucketing also writes the large-bucket GEMM's token-tile table (one for both GEMMs)
   p.bk.tiles = pf_up || pf_down ? p.tiles : nullptr;
   p.bk.half_tiles = pf_up && pf_down && moe::prefill_half_tiles(P, slots, gate, down);
@@ -637,7 +637,7 @@ int moe_switch_mlp_relu2(const moe_qweight* up, const moe_qweight* down, const u
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int E = up->experts;
   const int slots = static_cast<int>(P < E ? P : E);
-  const bool pf1_ = moe::use_prefill(P, slots, up, nullptr), pf2_ = moe::use_prefill(P, slots, down, nullptr);
+  const bool pf1_ = moe::use_prefill(P, slots, up, nullptr, T), pf2_ = moe::use_prefill(P, slots, down, nullptr);
   p.bk.tiles = pf1_ || pf2_ ? p.tiles : nullptr;
   st = moe::bucket(inds, T, k, E, p.bk, p.bucket_ws, p.bucket_ws_bytes, s);
   if (st != MOE_OK) return st;
@@ -722,7 +722,7 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   const bool rq_large = qrouter && moe::use_prefill(T, 1, &d->router_q, nullptr);
   const bool sh_up_large = d->shared_intermediate > 0 && moe::use_prefill(T, 1, &d->shared_gate, &d->shared_up);
   const bool sh_down_large = d->shared_intermediate > 0 && moe::use_prefill(T, 1, &d->shared_down, nullptr);
-  const bool pf_up = moe::use_prefill(P, slots, &d->gate, &d->up);
+  const bool pf_up = moe::use_prefill(P, slots, &d->gate, &d->up, T);
   const bool pf_down = moe::use_prefill(P, slots, &d->down, nullptr);
   // A shared expert of the routed experts' shape runs in their launches, its T
   // rows as one more expert's: the launches of one expert alone leave most CUs
@@ -750,8 +750,7 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   // when gate|up runs the large-bucket GEMM, the bf16 router projection (which
   // reads every row of x anyway) also writes the group sums of x that GEMM needs
   // (groups of whole 64-wide K steps; groups of 32 take the group-sum pass)
-  const bool fuse_sums = !qrouter && d->gate.group_size % 64 == 0 && moe::router_tile32(T, d->hidden) &&
-                         moe::use_prefill(P, slots, &d->gate, &d->up);
+  const bool fuse_sums = !qrouter && d->gate.group_size % 64 == 0 && moe::router_tile32(T, d->hidden) && pf_up;
   const moe::RouterGroupSums sums{reinterpret_cast<uint16_t*>(p.gsum), d->gate.group_size,
                                   moe::prefill_gsum_stride(&d->gate) / 16,
                                   sh_f32 || moe::prefill_f32_sums(&d->gate)};

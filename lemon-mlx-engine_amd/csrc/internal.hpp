@@ -257,7 +257,10 @@ int prefill_gsum_stride(const moe_qweight* w);
 bool prefill_f32_sums(const moe_qweight* w);
 int64_t prefill_tall_tile_ints(int64_t P, int E);  // tiles of up to 128 rows
 int64_t prefill_tile_ints(int64_t P, int E);       // either tiling
-bool use_prefill(int64_t P, int slots, const moe_qweight* w0, const moe_qweight* w1);
+// Whether P rows over at most `slots` non-empty experts run the large-bucket
+// GEMM.  x_rows = rows of x that they are gathered from (-1: at most P, or
+// rows named by the caller's indices, see PrefillScratch::far).
+bool use_prefill(int64_t P, int slots, const moe_qweight* w0, const moe_qweight* w1, int64_t x_rows = -1);
 // Whether grouped_qmm's gate|up launch for these arguments can route a single
 // token itself (pf.route): one token (P = k = slots), 4-bit codes with x in
 // pair K order, the per-16-row kernel with K split over four waves, E <= 512.

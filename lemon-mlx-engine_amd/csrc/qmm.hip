@@ -1146,10 +1146,13 @@ int64_t prefill_wgs(int64_t P, int slots, const moe_qweight* w0, bool glu) {
 // shape, measured: at 8 rows both paths take the same time, at 16 the GEMM
 // takes 0.6x the per-16-row kernel's, at 64 rows 0.42x), unless it would get
 // so few workgroups that most CUs idle (a shared expert at a few dozen tokens:
-// one expert's token tile times a handful of column tiles).
-bool use_prefill(int64_t P, int slots, const moe_qweight* w0, const moe_qweight* w1) {
+// one expert's token tile times a handful of column tiles), and where its
+// 32-bit byte offsets reach every row of x (below 4 GiB; the per-16-row kernel
+// has 64-bit ones).
+bool use_prefill(int64_t P, int slots, const moe_qweight* w0, const moe_qweight* w1, int64_t x_rows) {
   return P >= 16 * static_cast<int64_t>(slots) && prefill_supported(w0, w1) &&
-         prefill_wgs(P, slots, w0, w1 != nullptr) >= kPrefillMinWgs;
+         prefill_wgs(P, slots, w0, w1 != nullptr) >= kPrefillMinWgs &&
+         (x_rows >= 0 ? x_rows : P) * static_cast<int64_t>(w0->K) * 2 < (int64_t{1} << 32);
 }
 
 bool gate_up_route_fits(int64_t P, int slots, const PrefillScratch& pf, const moe_qweight* gate,
@@ -1160,7 +1163,7 @@ bool gate_up_route_fits(int64_t P, int slots, const PrefillScratch& pf, const mo
   if (P != k || slots != k || k > 16 || E > 512 || E != gate->experts) return false;
   // the partial sums of the logits: every load of a lane at once (token_logits_from_partials)
   if (ks < 1 || ks * ((E + 63) / 64) > 32) return false;
-  if (use_prefill(P, slots, gate, up)) return false;
+  if (use_prefill(P, slots, gate, up, 1)) return false;
   const int ksplit = gqmm_ksplit(P, slots, gate);
   return ksplit == 4 && !gqmm_sreg(gate, true, ksplit);
 }
@@ -1184,7 +1187,7 @@ int grouped_qmm(const uint16_t* x, const int32_t* row_in, const int32_t* row_out
   if (slots == 0) return MOE_OK;
   // Large buckets (prefill): the LDS-staged GEMM.  Small buckets (decode):
   // the per-16-row kernel below.
-  if (pf && !pf->gemv_only && use_prefill(P, slots, w0, w1))
+  if (pf && !pf->gemv_only && use_prefill(P, slots, w0, w1, pf->x_rows))
     return grouped_gemm_prefill(x, row_in, row_out, *pf, offsets, w0->experts, P, slots, w0, w1, out, stream);
   // 4-bit: activations already in pair K order (gate|up: the copy the router
   // projection wrote; down: h written in that order by gate|up)

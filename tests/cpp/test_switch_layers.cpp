@@ -42,6 +42,10 @@
 #include "safetensors.hpp"
 #include "switch_layers.hpp"
 
+namespace moe {
+bool use_prefill(int64_t P, int slots, const moe_qweight* w0, const moe_qweight* w1, int64_t x_rows = -1);
+}
+
 using namespace mlx_lm::mi355x;
 
 namespace {
@@ -267,6 +271,22 @@ TEST_CASE(validation_before_device, "cpu") {
   REQUIRE_THROWS_AS(moe_route(array({0, 8}, Dtype::float32), 2), std::invalid_argument);
   REQUIRE_THROWS_AS(array({0, 4}, Dtype::bfloat16).reshape({5}), std::invalid_argument);
   REQUIRE_THROWS_AS(SwitchLinear(0, 32, 4), std::invalid_argument);
+}
+
+// The library's rule for its large-bucket GEMM (csrc/internal.hpp): the rows of x end below 4 GiB, which
+// its 32-bit offsets reach; gate|up counts the T rows of x, not the T k pairs.
+TEST_CASE(large_bucket_gemm_rows, "cpu") {
+  for (const int bits : {4, 6, 8})
+    for (const int gs : {32, 64, 128}) {
+      const auto* p = reinterpret_cast<const uint32_t*>(0x10000);  // never dereferenced
+      const auto* h = reinterpret_cast<const uint16_t*>(0x10000);
+      const moe_qweight w{p, h, h, 8, 4096, 14336, gs, bits, nullptr};
+      const int64_t most = ((int64_t{1} << 32) - 1) / (2 * 14336);
+      REQUIRE(moe::use_prefill(most, 8, &w, nullptr));
+      REQUIRE(!moe::use_prefill(most + 1, 8, &w, nullptr));
+      REQUIRE(moe::use_prefill(8 * most, 8, &w, &w, most));
+      REQUIRE(!moe::use_prefill(8 * most, 8, &w, &w, most + 1));
+    }
 }
 
 // ---- checkpoint reading (json.hpp, safetensors.hpp, quantize_utils.hpp) -----------

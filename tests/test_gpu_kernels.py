@@ -353,6 +353,19 @@ def test_gather_qmm_whole_group_sums(bits, gs):
     assert (got == 0).all()
 
 
+def test_gather_qmm_rows_of_4gib():
+    """2^20 + 3 gathered rows of 4 KiB: more than the large-bucket GEMM addresses, so the per-16-row kernel
+    takes them, with the bytes it gives for a few of them."""
+    E, N, K, n, src = 8, 256, 2048, (1 << 20) + 3, 8
+    q = dqw(W.make_qweight(66, 2, E, N, K, 0.02, 64, 6))
+    x = dbf(W.normal_bf16(66, 100, src * K, 1.0).reshape(src, K))
+    rng = np.random.default_rng(66)
+    lhs, rhs = rng.integers(0, src, n), rng.integers(0, E, n)
+    got = moe.gather_qmm(x, q, di32(lhs), di32(rhs))
+    few = moe.gather_qmm(x, q, di32(np.repeat(np.arange(src), E)), di32(np.tile(np.arange(E), src)))
+    assert torch.equal(got, few[di32(lhs * E + rhs).long()])
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 def test_gather_qmm_tile_classes(bits):
     """Bucket remainders (mod 128 rows) of 0, 1, 32, 33, 64, 65, 96, 97 and 127
