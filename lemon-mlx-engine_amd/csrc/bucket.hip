@@ -42,6 +42,7 @@ __global__ __launch_bounds__(256) void bucket_count_kernel(const uint32_t* __res
                                                           int64_t P, int E,
                                                           int* __restrict__ cnt, int chunk, BucketOut o) {
   extern __shared__ int hist[];
+  if (o.far && blockIdx.x == 0 && threadIdx.x == 0) *o.far = 0;  // (the scatter launch sets it)
   for (int x = threadIdx.x; x < E; x += 256) hist[x] = 0;
   __syncthreads();
   const int64_t b0 = static_cast<int64_t>(blockIdx.x) * chunk;

@@ -82,7 +82,9 @@ __device__ __forceinline__ void write_sorted(uint32_t i, int pos, int k, const B
   if (o.sorted_token) o.sorted_token[pos] = static_cast<int32_t>(i / static_cast<uint32_t>(k));
   if (o.in_rows) {
     const uint32_t M = static_cast<uint32_t>(o.M), b = M == 1 ? i : i / M;
-    o.in_rows[pos] = static_cast<int32_t>((o.lhs ? o.lhs[b] : b) * M + (i - b * M));
+    const uint32_t row = (o.lhs ? o.lhs[b] : b) * M + (i - b * M);
+    o.in_rows[pos] = static_cast<int32_t>(row);
+    if (o.far && row >= o.far_row) *o.far = 1;
   }
 }
 
@@ -203,6 +205,7 @@ __device__ void bucket_fused_body(const uint32_t* __restrict__ inds, int64_t P, 
   int* offs = tot + E;              // [E+1]
   int* wcnt = offs + E + 1;         // [NW][E]
   int* sp = wcnt + NW * E;          // [P]
+  if (o.far && threadIdx.x == 0) *o.far = 0;
   const int lane = lane_id(), wave = threadIdx.x >> 6;
   const int rounds = (static_cast<int>(P) + NW * 64 - 1) / (NW * 64);
   const int i0 = wave * rounds * 64 + lane;

@@ -424,7 +424,7 @@ static moe::Carve gqmm_layout(void* ws, int64_t n, int32_t E, int32_t gstride, i
   *perm = c.take<int32_t>(n);
   *offsets = c.take<int32_t>(E + 1);
   *active = c.take<int32_t>(4 * static_cast<int64_t>(E));
-  *num_active = c.take<int32_t>(1);
+  *num_active = c.take<int32_t>(2);  // [1]: BucketOut::far
   *in_rows = c.take<int32_t>(n);
   *tiles = c.take<int32_t>(moe::prefill_tall_tile_ints(n, E));
   *gsum = c.take<float>(n * gstride);
@@ -476,9 +476,14 @@ int moe_gather_qmm(const uint16_t* x, const moe_qweight* w, const uint32_t* lhs,
   const bool pf_tiles = pf_ok && moe::use_prefill(n, slots, w, nullptr);
   if (pf_tiles) o.tiles = tiles;
   set_gather_pairs(o, lhs, M, inr, out, w->N);
+  if (pf_tiles && lhs) {  // rows of x that 32-bit byte offsets do not reach
+    o.far = na + 1;
+    o.far_row = static_cast<uint32_t>(((int64_t{1} << 32) - 1) / (2 * static_cast<int64_t>(w->K)));
+  }
   st = moe::bucket(rhs, n, 1, w->experts, o, bws, bb, s);
   if (st != MOE_OK) return st;
   moe::PrefillScratch pf{tiles, gsum, -1};
+  pf.far = o.far;
   pf.tiles_ready = pf_tiles;
   return moe::grouped_qmm(x, inr, perm, offs, act, na, slots, n, pf_ok ? &pf : nullptr, w, nullptr, out, s);
 }

@@ -70,6 +70,9 @@ struct BucketOut {
   int M = 1;
   const uint32_t* lhs = nullptr;
   int32_t* in_rows = nullptr;     // optional [P]: sorted position -> input row
+  // optional, with in_rows: [1] = whether an input row is far_row or more
+  int32_t* far = nullptr;
+  uint32_t far_row = 0;
   // optional: row i of zero_out [P, zero_N] is zeroed for a pair whose expert
   // is out of range (it is in no bucket, so no other kernel writes its row)
   uint16_t* zero_out = nullptr;
@@ -237,6 +240,8 @@ struct PrefillScratch {
   // large-bucket GEMM: fp32 group sums (gsum, and next_gsum where written here)
   // also where the weights do not ask for them (prefill_f32_sums)
   bool f32_sums = false;
+  // device flag of the bucketing (BucketOut::far): rows of x past 4 GiB
+  const int32_t* far = nullptr;
 };
 constexpr int kOneExpertSlots = 64;
 inline int one_expert_slots(int64_t P) { return static_cast<int>(std::min<int64_t>((P + 15) / 16, kOneExpertSlots)); }

@@ -95,6 +95,7 @@ struct PArgs {
   // projection, in the xhl layout (nch chunks of 2 bf16 planes), groups of gs
   uint16_t* hsum;
   int hsum_nch, hsum_gs, hsum_G;
+  const int32_t* far;       // device flag: != 0, some input row lies past 4 GiB of x (NULL: none)
   int hsum_f32;             // the sums of h as fp32 (the next projection's launch is F32S)
   int out_p8;               // GLU: write h in the pair K order (see pair_order)
   int act;                  // GLU: moe_activation of h = act(gate, up)
@@ -278,8 +279,9 @@ constexpr int prefill_lds_bytes() {
 // compiled (the selector's other branches, inlined into every tile height's
 // unrolled epilogue, doubled the kernel's code and cost ~4 % of gate|up).
 // G32: groups of 32, two per K step (another K order, below, and two folds).
-// F32S: whole fp32 group sums and a dividing SiLU (file header).
-template <int BITS, bool GLU, int MT, bool PAIRS, bool GACT, bool G32, bool F32S>
+// F32S: whole fp32 group sums and a dividing SiLU (file header).  ROWS64:
+// 64-bit row offsets into x.
+template <int BITS, bool GLU, int MT, bool PAIRS, bool GACT, bool G32, bool F32S, bool ROWS64>
 __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const int e, const int row0,
                                              const int rows, const int ntile) {
   constexpr int BM = 32 * MT;
@@ -326,16 +328,20 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
   //      and the step's offset in a scalar register ----
   // activation block j of this wave = tile rows 8*(wave + 4j) .. +7, 128
   // bytes each; lane -> row + lane/8, LDS slot lane%8 holds 16-byte chunk
-  // slot ^ ((row / 2) % 8).  Offsets into x fit 32 bits (checked on the host).
+  // slot ^ ((row / 2) % 8).  Offsets into x fit 32 bits (use_prefill) or,
+  // with ROWS64, each lane carries 64-bit addresses.
   const __amdgpu_buffer_rsrc_t xrs = raw_rsrc(a.x);
   uint32_t aoff[MT];
+  const uint8_t* asrc[MT];
   uint32_t zrow[MT];  // group-sum row of the same tile row (input row, or sorted position)
 #pragma unroll
   for (int j = 0; j < MT; ++j) {
     const int r = 8 * (wave + 4 * j) + (lane >> 3);
     const int pos = row0 + min(r, rows - 1);
     const uint32_t xr = static_cast<uint32_t>(a.row_in ? a.row_in[pos] : pos);
-    aoff[j] = xr * static_cast<uint32_t>(a.K) * 2u + 16u * static_cast<uint32_t>((lane & 7) ^ ((r >> 1) & 7));
+    const uint32_t au = 16u * static_cast<uint32_t>((lane & 7) ^ ((r >> 1) & 7));
+    if constexpr (ROWS64) asrc[j] = reinterpret_cast<const uint8_t*>(a.x) + static_cast<int64_t>(xr) * a.K * 2 + au;
+    else aoff[j] = xr * static_cast<uint32_t>(a.K) * 2u + au;
     zrow[j] = a.gsum_by_pos ? static_cast<uint32_t>(pos) : xr;
   }
   // code chunk q of this wave's 64 rows (bytes 64q .. 64q+63 of each) goes to
@@ -379,7 +385,10 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
     const uint32_t kc = static_cast<uint32_t>(min(ks, KS - 1));
     uint8_t* sb = lds + stage * kABytes;
 #pragma unroll
-    for (int j = 0; j < MT; ++j) buffer_load_lds16(xrs, aoff[j], kc * 128u, sb + (wave + 4 * j) * 1024);
+    for (int j = 0; j < MT; ++j) {
+      if constexpr (ROWS64) load_lds16(asrc[j] + kc * 128u, sb + (wave + 4 * j) * 1024);
+      else buffer_load_lds16(xrs, aoff[j], kc * 128u, sb + (wave + 4 * j) * 1024);
+    }
   };
   auto issue_b = [&](int q) {
     const uint32_t qc = static_cast<uint32_t>(min(q, NCH - 1));
@@ -930,14 +939,32 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_prefill_kernel(const
       a.lb[m] = a.sh.lb[m];
     }
   }
+  // rows named by the caller's indices (gather_qmm: natural order, no GLU) may
+  // lie anywhere in x: bodies with 64-bit row offsets where the bucketing found
+  // one past 4 GiB.  (For every such launch they cost 40.5 -> 50.4 us at Qwen3's
+  // up projection, 4 bits, T = 256: with global in place of buffer loads the
+  // compiler drains all of them before the group sums' LDS reads.)
+  if constexpr (!GLU && !PAIRS) {
+    if (a.far && *a.far != 0) {
+      if (slot < cnt.x)
+        prefill_tile<BITS, GLU, 4, PAIRS, GACT, G32, F32S, true>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+      else if (slot < nlong)
+        prefill_tile<BITS, GLU, 3, PAIRS, GACT, G32, F32S, true>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+      else if (slot < nlong + cnt.z)
+        prefill_tile<BITS, GLU, 2, PAIRS, GACT, G32, F32S, true>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+      else
+        prefill_tile<BITS, GLU, 1, PAIRS, GACT, G32, F32S, true>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+      return;
+    }
+  }
   if (slot < cnt.x)
-    prefill_tile<BITS, GLU, 4, PAIRS, GACT, G32, F32S>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+    prefill_tile<BITS, GLU, 4, PAIRS, GACT, G32, F32S, false>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
   else if (slot < nlong)
-    prefill_tile<BITS, GLU, 3, PAIRS, GACT, G32, F32S>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+    prefill_tile<BITS, GLU, 3, PAIRS, GACT, G32, F32S, false>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
   else if (slot < nlong + cnt.z)
-    prefill_tile<BITS, GLU, 2, PAIRS, GACT, G32, F32S>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+    prefill_tile<BITS, GLU, 2, PAIRS, GACT, G32, F32S, false>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
   else
-    prefill_tile<BITS, GLU, 1, PAIRS, GACT, G32, F32S>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
+    prefill_tile<BITS, GLU, 1, PAIRS, GACT, G32, F32S, false>(a, lds, tinfo.x, tinfo.y, tinfo.z, ntile);
 }
 
 // xhl[r] = the group sums X[g] (fp32) of row src(r) as bf16 hi and lo parts,
@@ -1114,7 +1141,7 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
   if (w1 && (!pf.xp || x_rows < 0)) return MOE_E_INVALID_ARG;
   const uint16_t* xin = w1 ? pf.xp : x;
   if (E > 1024) return MOE_E_UNSUPPORTED;
-  // the kernel addresses x with 32-bit byte offsets
+  // the kernel addresses x, and the group sums of P rows, with 32-bit byte offsets (use_prefill)
   if ((x_rows >= 0 ? x_rows : P) * static_cast<int64_t>(w0->K) * 2 >= (int64_t{1} << 32)) return MOE_E_UNSUPPORTED;
   const int gstride = prefill_gsum_stride(w0);
   const bool f32 = pf.f32_sums || prefill_f32_sums(w0);
@@ -1149,6 +1176,7 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
   a.xhl = reinterpret_cast<const uint16_t*>(gsum);
   a.nch = gstride / 16;
   a.gsum_by_pos = by_pos ? 1 : 0;
+  a.far = pf.far;
   a.tiles = tiles;
   a.w[0] = w0->w;
   a.s[0] = w0->scales;

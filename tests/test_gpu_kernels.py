@@ -353,6 +353,23 @@ def test_gather_qmm_whole_group_sums(bits, gs):
     assert (got == 0).all()
 
 
+@pytest.mark.parametrize("bits,gs", [(4, 64), (6, 64), (8, 64), (4, 32), (6, 32), (8, 32)])
+def test_gather_qmm_rows_past_4gib(bits, gs):
+    """Rows of x named by lhs beyond 4 GiB (x: 2^20 + 200 rows of 4 KiB): the same bytes as from a small x
+    that holds these rows.  The rows that the offsets' low 32 bits name hold other values."""
+    E, N, K, batch, far = 4, 2048, 2048, 200, 1 << 20
+    q = dqw(W.make_qweight(bits + 60, 2, E, N, K, 0.02, gs, bits))
+    rng = np.random.default_rng(bits)
+    rhs = di32(rng.integers(0, E, batch))
+    small = dbf(W.normal_bf16(bits, 100, batch * K, 1.0).reshape(batch, K))
+    x = torch.empty((far + batch, K), dtype=torch.bfloat16, device=DEV)
+    x[:batch] = 1.0
+    x[far:] = small
+    lhs = rng.permutation(batch)
+    got = moe.gather_qmm(x, q, di32(lhs + far), rhs)
+    assert torch.equal(got, moe.gather_qmm(small, q, di32(lhs), rhs))
+
+
 def test_gather_qmm_rows_of_4gib():
     """2^20 + 3 gathered rows of 4 KiB: more than the large-bucket GEMM addresses, so the per-16-row kernel
     takes them, with the bytes it gives for a few of them."""
