@@ -741,7 +741,9 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   const bool sh_shape = d->shared_intermediate > 0 && d->activation == MOE_ACT_SWIGLU &&
                         moe::shared_fits(d->gate, d->shared_gate) && moe::shared_fits(d->up, d->shared_up) &&
                         moe::shared_fits(d->down, d->shared_down);
-  const bool sh_large = sh_shape && pf_up && pf_down && E < 1024 && p.tiles_all && p.sh_hsum;
+  const bool sh_large = sh_shape && pf_up && pf_down && E < 1024 && p.tiles_all && p.sh_hsum &&
+                        moe::shared_fits_prefill(d->gate, &d->up, d->shared_gate, &d->shared_up) &&
+                        moe::shared_fits_prefill(d->down, nullptr, d->shared_down, nullptr);
   const bool sh_small = sh_shape && !pf_up && !pf_down && !sh_up_large && !sh_down_large;
   const bool sh_merged = sh_large || sh_small;
   // rows that would not run the large-bucket GEMM by themselves keep the

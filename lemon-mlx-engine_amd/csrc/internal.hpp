@@ -201,6 +201,12 @@ struct SharedRows {
 // Whether the projection s of the shared expert can run in the launch of the
 // routed projection w
 bool shared_fits(const moe_qweight& w, const moe_qweight& s);
+// Whether the large-bucket GEMM reads w's scales and biases in 16-byte loads of
+// 8 groups (else in dwords).  A launch reads all its weights one way.
+bool prefill_wide_scales(const moe_qweight& w);
+// Whether shared projections s0 (and s1) that fit may also run in the large-bucket
+// launch of w0 (and w1): not where their scales would take its reads to dwords.
+bool shared_fits_prefill(const moe_qweight& w0, const moe_qweight* w1, const moe_qweight& s0, const moe_qweight* s1);
 
 struct PrefillScratch {
   int32_t* tiles;   // [prefill_tile_ints(P, E)] token tile table

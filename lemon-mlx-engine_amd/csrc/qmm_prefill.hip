@@ -1123,6 +1123,16 @@ bool shared_fits(const moe_qweight& w, const moe_qweight& s) {
          (reinterpret_cast<uintptr_t>(s.w) & 15u) == 0 && (s.biases == nullptr) == (w.biases == nullptr);
 }
 
+bool prefill_wide_scales(const moe_qweight& w) {
+  auto al16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  return (w.K / w.group_size) % 8 == 0 && al16(w.scales) && (!w.biases || al16(w.biases));
+}
+
+bool shared_fits_prefill(const moe_qweight& w0, const moe_qweight* w1, const moe_qweight& s0, const moe_qweight* s1) {
+  return !(prefill_wide_scales(w0) && (!w1 || prefill_wide_scales(*w1))) ||
+         (prefill_wide_scales(s0) && (!s1 || prefill_wide_scales(*s1)));
+}
+
 // offsets [E+1] on device; tiles: prefill_tile_ints(P, E) ints of scratch
 // (tiles_ready: already built from these offsets);
 // gsum: scratch of max(x_rows, P) * prefill_gsum_stride(w0) 4-byte words.
@@ -1183,13 +1193,12 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
   a.b[0] = w0->biases;
   a.lb[0] = w0->linear_bias;
   a.lb[1] = w1 ? w1->linear_bias : nullptr;
-  auto al16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  bool wide = (w0->K / w0->group_size) % 8 == 0 && al16(w0->scales) && (!w0->biases || al16(w0->biases));
+  bool wide = prefill_wide_scales(*w0);
   if (w1) {
     a.w[1] = w1->w;
     a.s[1] = w1->scales;
     a.b[1] = w1->biases;
-    wide = wide && al16(w1->scales) && (!w1->biases || al16(w1->biases));
+    wide = wide && prefill_wide_scales(*w1);
   }
   a.N = w0->N;
   a.K = w0->K;
@@ -1226,7 +1235,7 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
       a.sh.s[m] = sw[m]->scales;
       a.sh.b[m] = sw[m]->biases;
       a.sh.lb[m] = sw[m]->linear_bias;
-      wide = wide && al16(sw[m]->scales) && (!sw[m]->biases || al16(sw[m]->biases));
+      wide = wide && prefill_wide_scales(*sw[m]);
     }
     a.wide_scales = wide ? 1 : 0;
     rows += sh.rows;

@@ -44,6 +44,7 @@
 
 namespace moe {
 bool use_prefill(int64_t P, int slots, const moe_qweight* w0, const moe_qweight* w1, int64_t x_rows = -1);
+bool shared_fits_prefill(const moe_qweight& w0, const moe_qweight* w1, const moe_qweight& s0, const moe_qweight* s1);
 }
 
 using namespace mlx_lm::mi355x;
@@ -287,6 +288,28 @@ TEST_CASE(large_bucket_gemm_rows, "cpu") {
       REQUIRE(moe::use_prefill(8 * most, 8, &w, &w, most));
       REQUIRE(!moe::use_prefill(8 * most, 8, &w, &w, most + 1));
     }
+}
+
+// The rule that lets a shared expert into the routed experts' large-bucket launches: never where its scales or
+// biases take the launch's reads from 16 bytes to dwords.
+TEST_CASE(shared_expert_scale_alignment, "cpu") {
+  const auto* p = reinterpret_cast<const uint32_t*>(0x10000);  // never dereferenced
+  const auto* h = reinterpret_cast<const uint16_t*>(0x10000);
+  const auto* h4 = h + 2;  // 4- but not 16-byte aligned
+  const moe_qweight w{p, h, h, 8, 1024, 1024, 64, 4, nullptr}, narrow{p, h4, h, 8, 1024, 1024, 64, 4, nullptr};
+  for (const auto* s : {h, h4})
+    for (const auto* b : {h, h4}) {
+      const moe_qweight sh{p, s, b, 1, 1024, 1024, 64, 4, nullptr}, whole{p, h, h, 1, 1024, 1024, 64, 4, nullptr};
+      const bool aligned = s == h && b == h;
+      REQUIRE(moe::shared_fits_prefill(w, nullptr, sh, nullptr) == aligned);
+      REQUIRE(moe::shared_fits_prefill(w, &w, sh, &whole) == aligned);
+      REQUIRE(moe::shared_fits_prefill(w, &w, whole, &sh) == aligned);
+      REQUIRE(moe::shared_fits_prefill(w, &narrow, sh, &whole));
+      REQUIRE(moe::shared_fits_prefill(narrow, nullptr, sh, nullptr));
+    }
+  // fewer than 8 groups a row: dwords for every weight
+  const moe_qweight w4{p, h, h, 8, 1024, 256, 64, 4, nullptr}, s4{p, h4, h4, 1, 1024, 256, 64, 4, nullptr};
+  REQUIRE(moe::shared_fits_prefill(w4, nullptr, s4, nullptr));
 }
 
 // ---- checkpoint reading (json.hpp, safetensors.hpp, quantize_utils.hpp) -----------

@@ -21,6 +21,7 @@ CPU checker on the same seeded inputs.
 * full size: offsets[E] = T*k, perm is a permutation, and a second run is
   bit-identical (the combine uses no atomics).
 """
+import ctypes
 import gc
 
 import numpy as np
@@ -347,6 +348,53 @@ def test_block_shared_whole_group_sums(bits, T):
     torch.cuda.synchronize()
     ref = O.moe_experts(host, x, aux["inds"].cpu().numpy().astype(np.uint32), aux["scores"].cpu().numpy())
     assert_close(hbf(out), ref, what="shared expert, whole group sums")
+
+
+def launch_names(blk, xd):
+    """Profiling labels of one forward's launches (the shared expert's own ones start with "shared_")."""
+    L = moe.lib()
+    moe.check(L.moe_profile_enable(1), "moe_profile_enable")
+    out = blk.forward(xd)
+    name, ms, names = ctypes.c_char_p(), ctypes.c_float(), []
+    for i in range(L.moe_profile_count()):
+        moe.check(L.moe_profile_record(i, ctypes.byref(name), ctypes.byref(ms)), "moe_profile_record")
+        names.append(name.value.decode())
+    moe.check(L.moe_profile_enable(0), "moe_profile_enable")
+    return out, names
+
+
+@pytest.mark.parametrize("part", [0, 1, 2])
+@pytest.mark.parametrize("what", ["scales", "biases"])
+def test_block_shared_unaligned_scales(part, what):
+    """A shared expert of the routed shape whose scales or biases are 4- but not 16-byte aligned keeps launches
+    of its own at prefill (in the routed experts' it would take every tile's scale reads to dwords), and the
+    block gives what it gives with aligned ones, up to the sums' order."""
+    cfg = W.MoeConfig("shared_unaligned", 63, 1024, 1024, 8, 2, moe.ROUTE_TOPK_PROBS, True, 4,
+                      shared_intermediate=1024)
+    host = W.make_layer(cfg)
+    x = W.make_tokens(cfg, 300)
+    xd = torch.from_numpy(x.view(np.int16)).to(DEV).view(torch.bfloat16)
+    blk = moe.MoeBlock.from_host(host, DEV)
+    ref, names = launch_names(blk, xd)
+    assert "shared_qmm_gate_up_swiglu" not in names and "gemm_gate_up_swiglu" in names
+    qw = [moe.QuantizedWeight.from_numpy(q.w, q.scales, q.biases, q.group_size, q.bits, DEV) for q in
+          (host.gate, host.up, host.down) + tuple(host.shared[:3])]
+    v = getattr(qw[3 + part], what)
+    moved = torch.empty(v.numel() + 2, dtype=v.dtype, device=DEV)[2:].view(v.shape)
+    moved.copy_(v)
+    assert moved.data_ptr() % 16 == 4
+    setattr(qw[3 + part], what, moved)
+    router = torch.from_numpy(host.router_weight.view(np.int16)).to(DEV).view(torch.bfloat16)
+    blk2 = moe.MoeBlock(cfg.router_params(), router, *qw[:3], None, tuple(qw[3:]) + (None,))
+    out, names = launch_names(blk2, xd)
+    assert "shared_qmm_gate_up_swiglu" in names and "gemm_gate_up_swiglu" in names
+    _, aux = blk.forward(xd, return_aux=True)
+    torch.cuda.synchronize()
+    inds, scores = aux["inds"].cpu().numpy().astype(np.uint32), aux["scores"].cpu().numpy()
+    want, terms = O.moe_experts(host, x, inds, scores, with_terms=True)
+    for o in (ref, out):
+        assert_close_block(hbf(o), want, terms, what=f"unaligned {what} of shared projection {part}",
+                           strict_frac=STRICT_FRAC)
 
 
 @pytest.mark.parametrize("act", [moe.ACT_GPTOSS, moe.ACT_GPTOSS_UPSTREAM])
