@@ -134,12 +134,12 @@ __device__ void scatter_subchunk(const uint32_t e, const int64_t i, int64_t P, i
 // offsets.  Requires E <= NT <= 1024; once per kernel.
 template <int NT>
 __device__ void finish_offsets(const int* tot, int64_t P, int E, int* offs_lds, const BucketOut& o) {
-  static_assert(NT <= 1024, "the packed counts below stay under 2^16");
+  static_assert(NT < 1 << 15, "the packed counts below (one per expert at most) stay under 2^15");
   const int e = threadIdx.x;
   const int c = e < E ? tot[e] : 0;
   int c4 = 0, c3 = 0, c2 = 0, c1 = 0;
   const int ct = e < E ? c : e == E ? o.sh_rows : 0;  // (the shared expert: tiles only; E < NT then)
-  tile_counts(ct, o.half_tiles, c4, c3, c2, c1);
+  tile_counts(ct, c4, c3, c2, c1);
   const int nz = c > 0 ? 1 : 0;
   // rows, 128-row tiles, non-empty | 32-row tiles, 96- | 64-row tiles
   int4 ex = make_int4(c, c4, nz | (c1 << 16), c3 | (c2 << 16)), n;
@@ -164,10 +164,24 @@ __device__ void finish_offsets(const int* tot, int64_t P, int E, int* offs_lds, 
     if (e == 0 && o.num_active) o.num_active[0] = na;
   }
   if (o.tiles) {  // the large-bucket GEMM's token-tile table
-    const int n3 = n.w & 0xffff, n2 = n.w >> 16, n1 = n.z >> 16;
-    if (e == 0) reinterpret_cast<int4*>(o.tiles)[0] = make_int4(n.y, n3, n2, n1);
+    int n4 = n.y, n3 = n.w & 0xffff, n2 = n.w >> 16, n1 = n.z >> 16;
+    int b4 = ex.y, b3 = ex.w & 0xffff, b2 = ex.w >> 16, b1 = ex.z >> 16;
+    // tiles of at most 64 rows: a 128-row one as two, a 96-row one as 64 + 32 (so
+    // their prefixes follow from the scan)
+    const bool half = o.half_max.tiles > 0 && 2 * (n4 + n3) + n2 + n1 <= o.half_max.tiles &&
+                      4 * n4 + 3 * n3 + 2 * n2 + n1 <= o.half_max.units;  // (uniform)
+    if (half) {
+      c1 += c3;
+      b1 += b3;
+      n1 += n3;
+      c2 += 2 * c4 + c3;
+      b2 += 2 * b4 + b3;
+      n2 += 2 * n4 + n3;
+      c4 = b4 = n4 = c3 = b3 = n3 = 0;
+    }
+    if (e == 0) reinterpret_cast<int4*>(o.tiles)[0] = make_int4(n4, n3, n2, n1);
     if (e <= E)
-      write_tiles(o.tiles, e < E ? e : -1, e < E ? ex.x : 0, ct, o.half_tiles, c4, c3, c2, c1, ex.y, ex.w & 0xffff, ex.w >> 16, ex.z >> 16, n.y, n3, n2);
+      write_tiles(o.tiles, e < E ? e : -1, e < E ? ex.x : 0, ct, half, c4, c3, c2, c1, b4, b3, b2, b1, n4, n3, n2);
   }
   __syncthreads();
 }

@@ -80,8 +80,8 @@ struct BlockPlan {
   int32_t* sh_offsets;
   int32_t* sh_active;
   int32_t* sh_num;
-  int32_t* tiles;      // token-tile table, tall tiles of the routed rows
-  int32_t* tiles_all;  // room for any table (prefill_tile_ints, with the shared expert), or NULL
+  int32_t* tiles;     // token-tile table of the routed rows
+  int32_t* tiles_sh;  // room for the table that also holds the shared expert's rows, or NULL
   int32_t* sh_tiles;
   float* gsum;
   float* hsum;  // group sums of h (written by the gate|up GEMM for down)
@@ -160,15 +160,11 @@ BlockPlan plan_block(const moe_block_desc* d, int64_t T, void* ws, size_t* total
   p.bk.offsets = c.take<int32_t>(E + 1);
   p.bk.active = c.take<int32_t>(4 * static_cast<int64_t>(E));
   p.bk.num_active = c.take<int32_t>(1);
-  // the tall tiling of the routed rows; the larger table (64-row tiles, the
-  // shared expert's T rows) takes the logits' place, which the routing has read
-  // before the bucketing writes the table: the workspace, and with it what fits
-  // the static scratch, stays the size of the tall one
-  const int64_t tall_ints = moe::prefill_tall_tile_ints(P, E), all_ints = moe::prefill_tile_ints(P + T, E + 1);
-  p.tiles = c.take<int32_t>(tall_ints);
-  p.tiles_all = all_ints <= tall_ints       ? p.tiles
-                : 2 * all_ints <= T * E     ? reinterpret_cast<int32_t*>(p.logits)
-                                            : nullptr;
+  p.tiles = c.take<int32_t>(moe::prefill_tile_ints(P, E));
+  // the table with the shared expert's T rows takes the logits' place, which the
+  // routing has read before the bucketing writes the table: the workspace, and
+  // with it what fits the static scratch, does not grow for it
+  p.tiles_sh = 2 * moe::prefill_tile_ints(P + T, E + 1) <= T * E ? reinterpret_cast<int32_t*>(p.logits) : nullptr;
   {
     int64_t g = T * moe::prefill_gsum_stride(&d->gate);
     g = std::max<int64_t>(g, P * moe::prefill_gsum_stride(&d->down));
@@ -203,7 +199,7 @@ BlockPlan plan_block(const moe_block_desc* d, int64_t T, void* ws, size_t* total
     p.sh_offsets = c.take<int32_t>(2);
     p.sh_active = c.take<int32_t>(4);
     p.sh_num = c.take<int32_t>(1);
-    p.sh_tiles = c.take<int32_t>(moe::prefill_tall_tile_ints(T, 1));
+    p.sh_tiles = c.take<int32_t>(moe::prefill_tile_ints(T, 1));
   }
   *total = c.size();
   return p;
@@ -426,7 +422,7 @@ static moe::Carve gqmm_layout(void* ws, int64_t n, int32_t E, int32_t gstride, i
   *active = c.take<int32_t>(4 * static_cast<int64_t>(E));
   *num_active = c.take<int32_t>(2);  // [1]: BucketOut::far
   *in_rows = c.take<int32_t>(n);
-  *tiles = c.take<int32_t>(moe::prefill_tall_tile_ints(n, E));
+  *tiles = c.take<int32_t>(moe::prefill_tile_ints(n, E));
   *gsum = c.take<float>(n * gstride);
   *bws_bytes = moe::bucket_workspace_bytes(n, E);
   *bws = c.raw(*bws_bytes);
@@ -494,7 +490,7 @@ static moe::Carve gmm_layout(void* ws, int64_t n, int32_t E, int32_t** perm, int
   *perm = c.take<int32_t>(n);
   *offsets = c.take<int32_t>(E + 1);
   *in_rows = c.take<int32_t>(n);
-  *tiles = c.take<int32_t>(moe::prefill_tall_tile_ints(n, E));
+  *tiles = c.take<int32_t>(moe::prefill_tile_ints(n, E));
   *bws_bytes = moe::bucket_workspace_bytes(n, E);
   *bws = c.raw(*bws_bytes);
   return c;
@@ -597,13 +593,13 @@ int moe_switch_glu(const moe_qweight* gate, const moe_qweight* up, const moe_qwe
   const bool pf_up = moe::use_prefill(P, slots, gate, up, T), pf_down = moe::use_prefill(P, slots, down, nullptr);
   // the bucketing also writes the large-bucket GEMM's token-tile table (one for both GEMMs)
   p.bk.tiles = pf_up || pf_down ? p.tiles : nullptr;
-  p.bk.half_tiles = pf_up && pf_down && moe::prefill_half_tiles(P, slots, gate, down);
+  p.bk.half_max = pf_up && pf_down ? moe::prefill_half_max(P, E, gate, down) : moe::HalfTiles{};
   st = moe::bucket(inds, T, k, E, p.bk, p.bucket_ws, p.bucket_ws_bytes, s);
   if (st != MOE_OK) return st;
   const bool fuse_hsum = pf_up && pf_down;
   moe::PrefillScratch pf1{p.tiles, p.gsum, T, false, fuse_hsum ? p.hsum : nullptr, down};
   pf1.tiles_ready = p.bk.tiles != nullptr;
-  pf1.half_tiles = p.bk.half_tiles;
+  pf1.half_max = p.bk.half_max;
   pf1.xp = p.xp;
   pf1.act = activation;
   // h in pair K order for a down GEMM that reads it so
@@ -615,7 +611,7 @@ int moe_switch_glu(const moe_qweight* gate, const moe_qweight* up, const moe_qwe
   // down writes each pair's row at its flat index t*k + j: out is [T, k, H]
   moe::PrefillScratch pf2{p.tiles, fuse_hsum ? p.hsum : p.gsum, P, fuse_hsum};
   pf2.tiles_ready = p.bk.tiles != nullptr;
-  pf2.half_tiles = p.bk.half_tiles;
+  pf2.half_max = p.bk.half_max;
   pf2.in_p8 = h_pairs;
   return moe::grouped_qmm(p.h, nullptr, p.bk.perm, p.bk.offsets, p.bk.active, p.bk.num_active, slots,
                           P, &pf2, down, nullptr, out, s);
@@ -741,7 +737,7 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   const bool sh_shape = d->shared_intermediate > 0 && d->activation == MOE_ACT_SWIGLU &&
                         moe::shared_fits(d->gate, d->shared_gate) && moe::shared_fits(d->up, d->shared_up) &&
                         moe::shared_fits(d->down, d->shared_down);
-  const bool sh_large = sh_shape && pf_up && pf_down && E < 1024 && p.tiles_all && p.sh_hsum &&
+  const bool sh_large = sh_shape && pf_up && pf_down && E < 1024 && p.tiles_sh && p.sh_hsum &&
                         moe::shared_fits_prefill(d->gate, &d->up, d->shared_gate, &d->shared_up) &&
                         moe::shared_fits_prefill(d->down, nullptr, d->shared_down, nullptr);
   const bool sh_small = sh_shape && !pf_up && !pf_down && !sh_up_large && !sh_down_large;
@@ -763,9 +759,9 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
                                   sh_f32 || moe::prefill_f32_sums(&d->gate)};
   // the bucketing also writes the large-bucket GEMM's token-tile table (one for both GEMMs)
   p.bk.sh_rows = sh_large ? static_cast<int>(T) : 0;
-  p.bk.half_tiles = pf_up && pf_down && p.tiles_all &&
-                    moe::prefill_half_tiles(P + p.bk.sh_rows, slots + (sh_large ? 1 : 0), &d->gate, &d->down);
-  if (sh_large || p.bk.half_tiles) p.tiles = p.tiles_all;
+  if (sh_large) p.tiles = p.tiles_sh;
+  if (pf_up && pf_down)
+    p.bk.half_max = moe::prefill_half_max(P + p.bk.sh_rows, sh_large ? E + 1 : E, &d->gate, &d->down);
   p.bk.tiles = pf_up || pf_down ? p.tiles : nullptr;
   // small batches: routing and bucketing in one workgroup, from the partial
   // sums of a router projection spread over many workgroups
@@ -834,7 +830,7 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   pf1.next_gsum = fuse_hsum ? p.hsum : nullptr;
   pf1.next_w = &d->down;
   pf1.tiles_ready = p.bk.tiles != nullptr;
-  pf1.half_tiles = p.bk.half_tiles;
+  pf1.half_max = p.bk.half_max;
   // (xp_ready false: the large-bucket GEMM writes x in pair order with the group sums)
   pf1.act = d->activation;
   pf1.f32_sums = sh_f32;
@@ -896,7 +892,7 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   // so the combine reads a token's k rows without a lookup
   moe::PrefillScratch pf2{p.tiles, fuse_hsum ? p.hsum : p.gsum, P, fuse_hsum};
   pf2.tiles_ready = p.bk.tiles != nullptr;
-  pf2.half_tiles = p.bk.half_tiles;
+  pf2.half_max = p.bk.half_max;
   pf2.in_p8 = h_pairs;
   pf2.f32_sums = sh_f32;
   if (sh_merged) pf2.shared = &sh2;

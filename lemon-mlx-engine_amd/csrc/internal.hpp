@@ -19,16 +19,7 @@ namespace moe {
 // rows); int4 1 + i = tile i {expert, first sorted row, rows, 0}: the n4
 // 128-row tiles (experts in order), then the n3 96-row, the n2 64-row and the
 // n1 32-row tiles.
-// half: tiles of at most 64 rows (c / 64 of them, and one of 64 or 32 rows for
-// the remainder), where the tall ones would leave CUs without a workgroup.
-__device__ __forceinline__ void tile_counts(int c, bool half, int& c4, int& c3, int& c2, int& c1) {
-  if (half) {
-    const int r = c & 63;
-    c4 = c3 = 0;
-    c2 = (c >> 6) + (r > 32 ? 1 : 0);
-    c1 = r > 0 && r <= 32 ? 1 : 0;
-    return;
-  }
+__device__ __forceinline__ void tile_counts(int c, int& c4, int& c3, int& c2, int& c1) {
   const int units = ((c & 127) + 31) >> 5;
   c4 = (c >> 7) + (units == 4 ? 1 : 0);
   c3 = units == 3 ? 1 : 0;
@@ -36,7 +27,8 @@ __device__ __forceinline__ void tile_counts(int c, bool half, int& c4, int& c3, 
   c1 = units == 1 ? 1 : 0;
 }
 // Expert e's entries (bucket at sorted row o0, c rows); b4/b3/b2/b1 = its
-// first index within each class, n4/n3/n2 = the class totals.
+// first index within each class, n4/n3/n2 = the class totals.  half: tiles of at
+// most 64 rows (HalfTiles; no c4, c3).
 __device__ __forceinline__ void write_tiles(int32_t* tiles, int e, int o0, int c, bool half, int c4, int c3, int c2,
                                             int c1, int b4, int b3, int b2, int b1, int n4, int n3, int n2) {
   int4* tab = reinterpret_cast<int4*>(tiles) + 1;
@@ -52,6 +44,14 @@ __device__ __forceinline__ void write_tiles(int32_t* tiles, int e, int o0, int c
   if (c1) tab[n4 + n3 + n2 + b1] = make_int4(e, rem0, r, 0);
 }
 
+// The token-tile table has tiles of at most 64 rows (of a bucket's c rows c / 64,
+// and one of 64 or 32 rows for the remainder) where at most `tiles` of them hold
+// every bucket, and at most 32 * `units` rows, each bucket's rounded up to 32
+// (prefill_half_max; tiles 0: never)
+struct HalfTiles {
+  int tiles = 0, units = 0;
+};
+
 struct BucketOut {
   int32_t* perm;           // [P]   sorted position -> flat pair index
   int32_t* inv_perm;       // [P]   flat pair index -> sorted position
@@ -62,7 +62,7 @@ struct BucketOut {
                            //       experts with a non-empty bucket, ascending, then rows = 0
   int32_t* num_active;     // [1]
   int32_t* tiles = nullptr;  // optional: the large-bucket GEMM's token-tile table (prefill_tile_ints)
-  bool half_tiles = false;  // the table's tiles have at most 64 rows (tile_counts)
+  HalfTiles half_max;
   int sh_rows = 0;  // > 0: the table also holds the tiles of the shared expert's
                     // sh_rows rows, as one more expert, numbered -1, from row 0
   // the gather_qmm / gather_mm pairs (k = 1): pair i = (b, m), b = i / M, takes
@@ -218,7 +218,7 @@ struct PrefillScratch {
   float* next_gsum = nullptr;
   const moe_qweight* next_w = nullptr;
   bool tiles_ready = false;  // tiles already holds the table for these offsets
-  bool half_tiles = false;   // the table holds tiles of at most 64 rows
+  HalfTiles half_max;        // that table's BucketOut::half_max
   // Pair K order (within 8 consecutive K values: 0, 4, 1, 5, 2, 6, 3, 7): the
   // GEMM reads its operand of 4-bit codes in it at 7 instead of 9 VALU
   // instructions per code word.  gate|up (w1 != NULL) reads its input from
@@ -259,15 +259,14 @@ int grouped_qmm(const uint16_t* x, const int32_t* row_in, const int32_t* row_out
                 int slots, int64_t P, const PrefillScratch* pf, const moe_qweight* w0,
                 const moe_qweight* w1, uint16_t* out, hipStream_t stream);
 bool prefill_supported(const moe_qweight* w0, const moe_qweight* w1);
-// Whether tiles of at most 64 rows suit the large-bucket GEMMs gate|up and down
-// of `rows` rows over at most `experts` non-empty experts.
-bool prefill_half_tiles(int64_t rows, int64_t experts, const moe_qweight* gate, const moe_qweight* down);
+// The most tiles of at most 64 rows that suit the large-bucket GEMMs gate|up and
+// down; they fit a table of prefill_tile_ints(P, E).
+HalfTiles prefill_half_max(int64_t P, int E, const moe_qweight* gate, const moe_qweight* down);
 int prefill_gsum_stride(const moe_qweight* w);
 // Whether the large-bucket GEMM keeps the group sums of w's input rows in fp32
 // (else as two bf16 parts).
 bool prefill_f32_sums(const moe_qweight* w);
-int64_t prefill_tall_tile_ints(int64_t P, int E);  // tiles of up to 128 rows
-int64_t prefill_tile_ints(int64_t P, int E);       // either tiling
+int64_t prefill_tile_ints(int64_t P, int E);
 // Whether P rows over at most `slots` non-empty experts run the large-bucket
 // GEMM.  x_rows = rows of x that they are gathered from (-1: at most P, or
 // rows named by the caller's indices, see PrefillScratch::far).

@@ -1021,7 +1021,7 @@ __global__ __launch_bounds__(1024) void make_tiles_kernel(const int32_t* __restr
   __shared__ int base[4][1025];
   const int t = threadIdx.x;
   int c4 = 0, c3 = 0, c2 = 0, c1 = 0;
-  if (t < E) tile_counts(offsets[t + 1] - offsets[t], false, c4, c3, c2, c1);
+  if (t < E) tile_counts(offsets[t + 1] - offsets[t], c4, c3, c2, c1);
   base[0][t] = c4;
   base[1][t] = c3;
   base[2][t] = c2;
@@ -1074,30 +1074,28 @@ bool prefill_f32_sums(const moe_qweight* w) { return w->bits == 6 || w->group_si
 // 4-byte words per row of the group-sum buffer: 32 bf16 or 16 fp32 per 16-group chunk
 int prefill_gsum_stride(const moe_qweight* w) { return (w->K / w->group_size + 15) / 16 * 16; }
 
-// header + at most P/128 + E' tiles of 128 rows and E' each of 64 and 32
-// rows, E' = min(E, P) non-empty experts; of at most 64 rows (prefill_half_tiles:
-// P/128 < kHalfTileWgs then), P/64 + 2 E'
-constexpr int64_t kHalfTileWgs = 512;
-int64_t prefill_tall_tile_ints(int64_t P, int E) { return 4 * (1 + P / 128 + 3 * std::min<int64_t>(E, P)); }
-int64_t prefill_tile_ints(int64_t P, int E) {
-  return prefill_tall_tile_ints(P, E) + 4 * std::min<int64_t>(P / 128 + 1, kHalfTileWgs);
-}
+// At most P/128 + E' tiles of 128 rows and E' each of 64 and 32 rows, E' =
+// min(E, P) non-empty experts
+static int64_t prefill_max_tiles(int64_t P, int E) { return P / 128 + 3 * std::min<int64_t>(E, P); }
+int64_t prefill_tile_ints(int64_t P, int E) { return 4 * (1 + prefill_max_tiles(P, E)); }
 
-// Tiles of at most 64 rows where the launch lasts about as long as its longest
-// tile: where the 128-row tiling gives both projections at most two workgroups
-// per CU (one round), and where hardly a bucket holds more than 64 rows.
-// Elsewhere the tall tile's fewer code expansions per row win.  Measured (us,
-// tall | half), workgroups of the wider projection in brackets: SwitchGLU, 1024
-// x 1024, E 32, k 4: T = 256 [320] 75 | 53, 777 [448] 88 | 67, 1024 [512] 91 |
-// 80, 2048 [768] 119 | 129; 2048 x 2048, E 8, k 2: T = 256 [192] 108 | 69, 1024
-// [384] 121 | 105, 2048 [640] 169 | 189; 512 x 1024, E 128, k 8: T = 300 (19 rows
-// per expert) 69 | 57, 500 (31 rows) 74 | 75; Qwen3 block T = 256 (16 rows) 143 |
-// 139, 500 (31 rows) 165 | 167.
-constexpr int kHalfTileRows = 20;  // rows per expert on average
-bool prefill_half_tiles(int64_t rows, int64_t experts, const moe_qweight* gate, const moe_qweight* down) {
-  const int64_t tiles = rows / 128 + experts;
-  return rows < kHalfTileRows * experts ||
-         (tiles * (gate->N / (kBN / 2)) <= kHalfTileWgs && tiles * (down->N / kBN) <= kHalfTileWgs);
+// Tiles of at most 64 rows where they give the two launches at most about two
+// workgroups per CU on average and little more work than the tall ones: the
+// launches then last about as long as their longest tile.  Beyond that the tall
+// tile's fewer code expansions per row win, at 8 bits sooner.  The bucketing
+// counts the tiles, so uneven loads count as they are.  Measured (SwitchGLU, us,
+// tall | half; even loads, then all rows in an eighth of the experts): 1024 x
+// 1024, E 32, k 4, 4 bits: T = 614 56 | 50, 64 | 49, T = 1024 70 | 72, 68 | 53, 6
+// bits T = 900 92 | 85, 90 | 66; 2048 x 2048, E 8, k 2: T = 512 103 | 68, T = 1126
+// 108 | 110 (uneven 118 | 110); 4096 x 1024, E 8, k 2, T = 1126 129 | 117; 2048 x
+// 768, E 128, k 8, T = 280 (mostly one tile a bucket: the same) 115 | 115, 84 |
+// 60.  Past the limits: 1024 x 512, E 64, k 6, T = 1300 64 | 78, 8 bits 67 | 94;
+// 8 bits, 1024 x 1024, T = 1024 73 | 82; 2048 x 512, E 512, k 10, T = 900, an
+// eighth busy 111 | 129.
+HalfTiles prefill_half_max(int64_t P, int E, const moe_qweight* gate, const moe_qweight* down) {
+  const int nt = gate->N / (kBN / 2) + down->N / kBN;  // workgroups of a tile
+  return {static_cast<int>(std::min<int64_t>(1040 / nt, prefill_max_tiles(P, E))),
+          2 * (gate->bits == 8 ? 720 : 900) / nt};
 }
 
 bool prefill_supported(const moe_qweight* w0, const moe_qweight* w1) {
@@ -1242,11 +1240,11 @@ int grouped_gemm_prefill(const uint16_t* x, const int32_t* row_in, const int32_t
     experts += 1;
   }
   // per XCD: an eighth of the 128- and 96-row tiles, then of the short ones
-  // (n4 + n3 <= P/128 + slots, n2 + n1 <= slots: one remainder tile per expert)
-  // (tiles of at most 64 rows: n2 <= rows/64 + experts, n1 <= experts)
+  // (n4 + n3 <= rows/128 + experts, n2 + n1 <= experts: one remainder tile per
+  // expert; where the table holds tiles of at most 64 rows alone, half_max.tiles)
   const int64_t nt = a.n_tiles;
-  const int64_t n_long = pf.half_tiles ? 0 : rows / 128 + experts;
-  const int64_t n_short = 2 * experts + (pf.half_tiles ? rows / 64 : 0);
+  const int64_t n_long = rows / 128 + experts;
+  const int64_t n_short = std::max<int64_t>(2 * experts, pf.half_max.tiles);
   const int64_t grid = 8 * ((n_long * nt + 7) / 8 + (n_short * nt + 7) / 8);
   if (grid > 0x7fffffffLL) return MOE_E_UNSUPPORTED;
   const unsigned g = static_cast<unsigned>(grid);

@@ -579,6 +579,30 @@ def test_switch_glu_half_tiles():
     _switch_glu_case(inds.size, 1, len(counts), 1024, 1024, 4, 64, False, inds=inds.reshape(-1, 1))
 
 
+@pytest.mark.parametrize("bits,skew,tiles", [(4, False, 75), (6, False, 75), (8, False, 60), (4, True, 86), (8, True, 75)])
+def test_switch_glu_tile_height_rule(bits, skew, tiles):
+    """Tiles of at most 64 rows up to the most that the rule takes (with 12 workgroups a tile: 86 tiles; 150 units
+    of 32 rows, 120 at 8 bits), tall ones from one tile more on: a row's output is the same bytes on both sides
+    (its sums do not depend on its tile's height), for even loads and for one large bucket beside 31 of one row."""
+    E, H, I = 32, 1024, 1024
+    rng = np.random.default_rng(bits)
+    q = [dqw(W.make_qweight(70 + bits, i, E, n, K, 0.02, 64, bits)) for i, (n, K) in enumerate(((I, H), (I, H), (H, I)))]
+    if skew:
+        counts = np.ones(E, np.int64)
+        counts[7] = 64 * (tiles - E + 1)
+    else:
+        counts = 64 * (tiles // E + (np.arange(E) < tiles % E)) - 5
+    assert (-(-counts // 64)).sum() == tiles
+    inds = np.concatenate([np.repeat(np.arange(E), counts), np.full(64, 7)])  # the last 64: one tile more
+    x = dbf(W.normal_bf16(bits, 100, inds.size * H, 1.0).reshape(-1, H))
+    order = rng.permutation(inds.size)
+    kept = order < inds.size - 64
+    few = moe.switch_glu(x[di32(order[kept]).long()], di32(inds[order[kept]][:, None]), *q)
+    many = moe.switch_glu(x[di32(order).long()], di32(inds[order][:, None]), *q)
+    assert torch.equal(few, many[di32(np.flatnonzero(kept)).long()])
+    assert bool(few.float().abs().amax(dim=(1, 2)).min() > 0)
+
+
 @pytest.mark.parametrize("T,k,E,H,I,bits,gs", [(300, 2, 4, 512, 256, 6, 64), (300, 2, 4, 512, 256, 6, 32),
                                                (301, 2, 4, 256, 768, 4, 32), (77, 2, 2, 512, 256, 8, 32)])
 def test_switch_glu_large_buckets_widths(T, k, E, H, I, bits, gs):
