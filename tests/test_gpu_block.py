@@ -363,6 +363,48 @@ def launch_names(blk, xd):
     return out, names
 
 
+SHARED_ROUTES = [  # E, k, H, T, linear biases, router bits, one launch with the routed experts
+    (8, 2, 1024, 1, True, None, True),     # routed in the gate|up kernel; down with the combine, the shared one's alone
+    (8, 2, 1024, 1, False, 8, True),       # quantized router: x in natural K order
+    (8, 2, 1024, 33, True, None, True),    # per-16-row kernel
+    (8, 2, 1024, 33, False, 8, True),
+    (8, 2, 1024, 300, True, None, True),   # large-bucket GEMM; the table lies where the logits did
+    (8, 2, 1024, 300, False, 8, True),     # x in pair order from the group-sum pass
+    (8, 2, 1024, 600, False, None, True),  # group sums from the router projection
+    (8, 1, 1024, 300, False, None, False), # top-1: no room for the group sums of the shared expert's h
+    (4, 4, 2048, 16, False, None, False),  # the table of all rows is larger than the logits,
+    (4, 4, 2048, 33, False, None, False),  # ... by one tile,
+    (4, 4, 2048, 34, False, None, True),   # ... as large
+]
+
+
+@pytest.mark.parametrize("E,k,H,T,lb,rbits,merged", SHARED_ROUTES)
+def test_block_shared_routes(E, k, H, T, lb, rbits, merged):
+    """A shared expert of the routed shape in the routed launches (linear biases on every projection, a
+    quantized router) and at the edges where the workspace has no room for that: outputs against the checker, and
+    the call without aux (logits in the workspace) gives the same bytes."""
+    cfg = W.MoeConfig("shared_routes", 64, H, 1024, E, k, moe.ROUTE_TOPK_PROBS, True, 4, shared_intermediate=1024,
+                      shared_gated=True)
+    host = W.make_layer(cfg, router_bits=rbits, linear_bias=lb)
+    if lb:
+        for i, q in enumerate(host.shared[:3]):
+            q.linear_bias = W.normal_bf16(cfg.seed, 200 + i, q.N, 0.1).reshape(1, q.N)
+    blk = moe.MoeBlock.from_host(host, DEV)
+    x = W.make_tokens(cfg, T)
+    xd = torch.from_numpy(x.view(np.int16)).to(DEV).view(torch.bfloat16)
+    out, aux = blk.forward(xd, return_aux=True)
+    plain, names = launch_names(blk, xd)
+    torch.cuda.synchronize()
+    own = {"shared_qmm_gate_up_swiglu", "shared_gemm_gate_up_swiglu"} & set(names)
+    assert bool(own) != merged, names
+    assert (hbf(plain) == hbf(out)).all()
+    inds, scores = aux["inds"].cpu().numpy().astype(np.uint32), aux["scores"].cpu().numpy()
+    ref, terms = O.moe_experts(host, x, inds, scores, with_terms=True)
+    # (biases: one more bf16 rounding of g, u and h)
+    extra = h_rounding_mag(O, host, x, inds, scores) if lb else None
+    assert_close_block(hbf(out), ref, terms, what=f"shared E={E} k={k} T={T}", strict_frac=STRICT_FRAC, extra=extra)
+
+
 @pytest.mark.parametrize("part", [0, 1, 2])
 @pytest.mark.parametrize("what", ["scales", "biases"])
 def test_block_shared_unaligned_scales(part, what):
@@ -449,13 +491,15 @@ def test_block_6bit_experts(T):
 
 @pytest.mark.timeout(600)
 @pytest.mark.parametrize("bits,gs,T", [(2, 64, 1), (3, 64, 1), (5, 64, 1), (2, 64, 64), (3, 64, 64), (5, 64, 64),
-                                       (3, 64, 600), (4, 32, 1), (4, 32, 64), (4, 32, 600), (8, 32, 8), (3, 32, 64)])
+                                       (3, 64, 600), (4, 32, 1), (4, 32, 64), (4, 32, 600), (8, 32, 8), (3, 32, 64),
+                                       (3, 32, 600)])
 def test_block_lowbit_experts(bits, gs, T):
     """Qwen3-30B-A3B shape with 2-, 3- and 5-bit experts and with group size 32 (MLX's other affine
     widths and group size; the reference's converter takes --bits and --group-size,
-    examples/convert.cpp:19-20): routing bit-exact and every output against the checker.  These run
-    on the per-16-row kernel at every bucket size (T = 600: ~37 rows a bucket, several token chunks
-    per wave); 4-bit gs 32 at T = 1 also runs the one-token down + combine kernel."""
+    examples/convert.cpp:19-20): routing bit-exact and every output against the checker.  2, 3 and 5
+    bits run on the per-16-row kernel at every bucket size (T = 600: ~37 rows a bucket, several token
+    chunks per wave), 4-bit gs 32 at T = 600 on the large-bucket GEMM; 4-bit gs 32 at T = 1 also runs the
+    one-token down + combine kernel."""
     import dataclasses
     _cache.clear()
     gc.collect()

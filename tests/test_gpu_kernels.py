@@ -146,7 +146,7 @@ def test_bucket_skewed_single_expert():
 def test_gather_qmm_group32(bits, E, N, K, batch):
     """Group size 32 (MLX's --group-size 32): the per-16-row kernel with one MFMA per group (each lane's
     K values of a block split into the two 32-wide groups), at every width; decode-sized buckets, a
-    bucket of 40 rows, one pair, and ~150 rows an expert (large buckets stay on this kernel)."""
+    bucket of 40 rows, one pair, and ~150 rows an expert (too few workgroups for the large-bucket GEMM)."""
     q = W.make_qweight(bits + 30, 2, E, N, K, 0.02, 32, bits)
     x = W.normal_bf16(bits + 30, 100, batch * K, 1.0).reshape(batch, 1, K)
     rhs = np.random.default_rng(batch + bits).integers(0, E, batch).astype(np.uint32)
@@ -256,12 +256,13 @@ def test_gather_pairs_bucketing(E, batch, M):
     assert torch.equal(out.float().cpu(), ref)
 
 
-@pytest.mark.parametrize("kind,batch", [("q4", 16), ("q4", 1000), ("q6", 40), ("dense", 16), ("dense", 1000)])
-def test_gather_out_of_range_experts(kind, batch):
+@pytest.mark.parametrize("kind,batch,N", [("q4", 16, 256), ("q4", 1000, 256), ("q6", 40, 256), ("dense", 16, 256),
+                                          ("dense", 1000, 256), ("q4", 1000, 2048), ("q6", 1000, 2048)])
+def test_gather_out_of_range_experts(kind, batch, N):
     """rhs entries >= E (outside the contract; the checker rejects them): those output rows are zeros,
-    the other rows equal the checker's on the valid pairs (per-16-row kernel at 16 and 40 pairs,
-    large-bucket GEMM / dense tiles at 1000)."""
-    E, N, K = 4, 256, 1024
+    the other rows equal the checker's on the valid pairs (per-16-row kernel at N = 256, large-bucket GEMM at
+    N = 2048, dense tiles)."""
+    E, K = 4, 1024
     rng = np.random.default_rng(batch + 7)
     rhs = rng.integers(0, E, batch).astype(np.uint32)
     bad = rng.permutation(batch)[: max(1, batch // 8)]
@@ -285,11 +286,12 @@ def test_gather_out_of_range_experts(kind, batch):
 
 
 @pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 8])
-@pytest.mark.parametrize("E,N,K,batch", [(8, 512, 2048, 16), (4, 256, 1024, 1000), (3, 40, 512, 9)])
+@pytest.mark.parametrize("E,N,K,batch", [(8, 512, 2048, 16), (4, 256, 1024, 1000), (3, 40, 512, 9),
+                                         (4, 2048, 512, 1000)])
 def test_gather_qmm_linear_bias(bits, E, N, K, batch):
     """SwitchLinear with a bias (switch_layers.cpp:111-114): bf16(bf16(x.W^T) + bias[rhs]) from the
-    epilogue of the per-16-row kernel (16 and 9 pairs; N = 40: a partial last tile) and of the
-    large-bucket GEMM (1000 pairs)."""
+    epilogue of the per-16-row kernel (N = 40: a partial last tile) and of the large-bucket GEMM
+    (N = 2048; 4, 6 and 8 bits)."""
     q = W.make_qweight(bits + 20, 2, E, N, K, 0.02, 64, bits)
     q.linear_bias = W.normal_bf16(bits, 10, E * N, 0.1).reshape(E, N)
     x = W.normal_bf16(bits, 100, batch * K, 1.0).reshape(batch, 1, K)
@@ -300,15 +302,18 @@ def test_gather_qmm_linear_bias(bits, E, N, K, batch):
 
 @pytest.mark.parametrize("bits", [2, 3, 4, 5, 6, 8])
 @pytest.mark.parametrize("E,N,K,batch,skew,gs", [
-    (4, 256, 512, 1000, False, 64),     # ~250 rows per expert: 256-row token tiles
+    (4, 256, 512, 1000, False, 64),     # ~250 rows per expert
     (8, 512, 768, 700, True, 64),       # one expert holds half the rows, others ragged
-    (2, 512, 1024, 130, False, 64),     # 64-row token tiles, partial last tile
-    (3, 256, 256, 5000, True, 64),      # many token tiles per expert
-    (2, 256, 1024, 600, False, 128),    # group size 128: two K steps per scale
+    (2, 512, 1024, 130, False, 64),
+    (3, 256, 256, 5000, True, 64),
+    (2, 256, 1024, 600, False, 128),
+    (8, 2048, 512, 700, True, 64),      # the GEMM: one expert holds half the rows
+    (3, 1024, 256, 5000, True, 64),     # many token tiles per expert
+    (4, 2048, 512, 600, False, 128),    # group size 128: two K steps per scale
 ])
 def test_gather_qmm_large_buckets(bits, E, N, K, batch, skew, gs):
-    """Large per-expert buckets take the LDS-staged GEMM path (prefill; 6-bit: the per-16-row
-    kernel over many token chunks)."""
+    """Large per-expert buckets: the per-16-row kernel over many token chunks where the GEMM would get fewer
+    than 64 workgroups (the first five) and at 2, 3 and 5 bits, else the LDS-staged GEMM."""
     q = W.make_qweight(bits + 10, 2, E, N, K, 0.02, gs, bits)
     x = W.normal_bf16(bits, 100, batch * K, 1.0).reshape(batch, 1, K)
     rng = np.random.default_rng(batch)
@@ -394,7 +399,7 @@ def test_gather_qmm_tile_classes(bits):
 
 def _tile_classes_case(bits, gs, K):
     counts = [128, 129, 160, 161, 192, 193, 224, 225, 255]
-    E, N = len(counts), 256
+    E, N = len(counts), 1024  # (at least 64 workgroups, from which the GEMM runs)
     q = W.make_qweight(bits + 30, 2, E, N, K, 0.02, gs, bits)
     rhs = np.repeat(np.arange(E, dtype=np.uint32), counts)
     batch = rhs.size
