@@ -174,7 +174,9 @@ BlockPlan plan_block(const moe_block_desc* d, int64_t T, void* ws, size_t* total
     }
     p.gsum = c.take<float>(g);
     // past the sums of x, where there is room (those of h are in hsum when the
-    // shared expert's are needed)
+    // shared expert's are needed): k times down's sums of a row at least gate's
+    // plus the shared down's.  A top-1 block has none, and its shared expert keeps
+    // launches of its own at prefill
     if (d->shared_intermediate > 0) {
       const int64_t sx = T * moe::prefill_gsum_stride(&d->gate);
       p.sh_hsum = ws && sx + T * moe::prefill_gsum_stride(&d->shared_down) <= g ? p.gsum + sx : nullptr;
@@ -729,7 +731,7 @@ int block_forward(const moe_block_desc* d, const uint16_t* x, int64_t T, uint16_
   // rows as one more expert's: the launches of one expert alone leave most CUs
   // idle (Qwen3-Next T = 1001: six of them, 65 us).  Whole blocks, separate |
   // merged (us): Qwen3-Next T = 1 36.5 | 31.1, 8 77 | 65, 128 199 | 188, 1001
-  // 389 | 346; DeepSeek-V3 T = 1 97 | 85, 64 834 | 793, 600 2074 | 1954.  On
+  // 389 | 351; DeepSeek-V3 T = 1 97 | 85, 64 834 | 793, 600 2074 | 1954.  On
   // the per-16-row kernel only while the shared rows would run there too (many
   // rows of one expert: the large-bucket GEMM by itself).  A launch has one
   // activation and the shared expert's is always SwiGLU, so routed experts with

@@ -24,13 +24,16 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // ring.  The 16-byte chunk c of row r sits at slot c ^ ((r / 4) % 4): the 16
 // lanes that a 128-bit LDS read serves per clock never share a bank.
 //
-// What bounds it: up to a hundred rows per expert the weights' HBM stream
-// (every weight is read once per token tile), with several hundred the LDS
-// reads beside the MFMAs ((MT + NT) KB per MT * NT MFMAs).  Measured on
-// [E 128, N 768, K 2048], k = 8, the whole gather_mm call: T = 1500 912 -> 128
-// us, T = 4096 2332 -> 205, T = 256 207 -> 104, T = 16 68 -> 61, T = 1 27.6 ->
-// 23.1, against a kernel without LDS whose waves read every weight row from
-// L2 again for each 32 tokens and awaited each step's loads before its MFMAs.
+// What bounds it: up to a few dozen rows per expert the weights' HBM stream
+// (every weight is read once per token tile).  At 94 rows (T = 1500 below) the
+// weights come at 3.5 TB/s, and by counters neither the MFMA pipe (busy 15 % of
+// the cycles) nor LDS (0.13 conflict cycles per instruction, 1 % of the waves'
+// time waiting for it) is what it waits for: the waves wait for loads and the
+// step's barrier 25 % of their time and to issue 62 %.  Measured on [E 128, N 768,
+// K 2048], k = 8, the whole gather_mm call (us): T = 1500 916 -> 116, T = 4096
+// 2427 -> 179, T = 256 194 -> 94, T = 16 57 -> 40, T = 1 23.8 -> 19.7, against a
+// kernel without LDS whose waves read every weight row from L2 again for each 32
+// tokens and awaited each step's loads before its MFMAs.
 struct GMArgs {
   const uint16_t* x;
   const int32_t* row_in;
@@ -246,6 +249,9 @@ int grouped_mm(const uint16_t* x, const int32_t* row_in, const int32_t* row_out,
   //   32 - 94:            [128, 768, 2048] 239 | 135 | 128 (94), [32, 1024, 1024] 43 | 27 | 38 (32)
   //   256 - 1024:         [128, 768, 2048] 459 | 240 | 205, [8, 2048, 4096] 556 | 258 | 245,
   //                       [32, 1024, 1024] 145 |  74 |  81 (K = 1024: the tile's fill and epilogue weigh more)
+  // (nearly even loads; 32-row tiles | 128 columns where an eighth of the experts
+  // hold all rows, the first shape: 4 rows per expert on average 32 | 25, 8: 44 |
+  // 27.  The kernel before took 54 and 81.)
   // so: 32-row tiles up to 8 rows per expert, 256 columns (half the LDS reads
   // per MFMA, two workgroups per CU) from 32 rows where K >= 2048 and the grid
   // still fills the CUs.

@@ -50,7 +50,8 @@
 //     other weight tile's row taken from the lane 32 apart (v_permlane32_swap).
 // LDS chunks are XOR-swizzled 16-byte units, so that the 16 lanes a 128-bit
 // LDS read serves per clock (64 banks of 4 bytes) never share a bank: keyed on
-// row / 2 for the 128-byte activation rows, row / 4 for the 64-byte code rows.
+// row / 2 for the 128-byte activation rows, row / 4 for the 64-byte code rows
+// (6-bit codes are not swizzled).
 //
 // K order.  Within a 64-wide step, lane half h (= lane/32) of the A and B
 // operands of substep s carries K = 32h + 8s + [0, 8): a lane's B operands for
@@ -59,9 +60,9 @@
 // of the first group and 2, 3 the same of the second, so each group is a chain
 // of two MFMAs with a fold of its own (twice the fold FMAs).
 //
-// Which calls: whole blocks at the Qwen3 shape, against the per-16-row kernel
-// (us): 6 bits T = 256 291 -> 201, T = 2048 1369 -> 413; groups of 32 at 4 bits
-// T = 256 291 -> 178, T = 2048 1501 -> 381, at 8 bits T = 2048 1727 -> 416.
+// Which calls: whole blocks at the Qwen3 shape, the per-16-row kernel | this
+// one (us, one box): 6 bits T = 256 250 | 190, T = 2048 1303 | 390; groups of 32
+// at 4 bits T = 256 271 | 169, T = 2048 1415 | 348, at 8 bits T = 2048 1594 | 376.
 //
 // Scheduling.  Blocks are numbered so that consecutive virtual tiles land on
 // the same XCD (the hardware deals workgroups round-robin over 8 XCDs): the N
@@ -81,7 +82,8 @@ struct PArgs {
                             // (F32S: 16 fp32 in the chunk's 64 bytes)
   int nch;                  // 16-group chunks per row (G rounded up to 16, / 16)
   int gsum_by_pos;          // xhl rows: 1 = sorted position, 0 = input row (as x)
-  const int32_t* tiles;     // [0] = token tile count; entry i at 4+4i: {expert, row0, rows, 0}
+  const int32_t* tiles;     // token-tile table (tile_counts / write_tiles): int4 [0] = {n4, n3, n2, n1},
+                            // [1 + i] = tile i {expert (-1: the shared one), row0, rows, 0}
   int n_tiles;              // 256-row (GLU: 128-column) tiles along N
   const uint32_t* w[2];
   const uint16_t* s[2];
@@ -366,9 +368,11 @@ __device__ __forceinline__ void prefill_tile(const PArgs& a, uint8_t* lds, const
   };
   uint8_t* bring = lds + kLdsA + wave * (kBSlots * kChunkBytes);
   // 6-bit: the 64 rows' 48-byte runs are 192 16-byte units, three per row; lane
-  // -> unit 64 i + lane of instruction i, stored in order (row pitch 48 bytes:
-  // the lanes' 8-byte reads spread over all banks).  A unit's row decides its
-  // matrix, so each lane carries its own address
+  // -> unit 64 i + lane of instruction i, stored in order.  At a row pitch of
+  // 48 bytes lanes l and l + 16 read the same banks: 1.5 conflict cycles per LDS
+  // instruction (counters, gate|up at the Qwen3 shape, T = 2048; 4 bits: 0.05), 3 %
+  // of the launch's cycles.  A unit's row decides its matrix, so each lane carries
+  // its own address
   const uint8_t* csrc[3] = {nullptr, nullptr, nullptr};
   if constexpr (BITS == 6) {
 #pragma unroll
