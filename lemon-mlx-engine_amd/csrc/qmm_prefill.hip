@@ -1086,20 +1086,30 @@ int64_t prefill_tile_ints(int64_t P, int E) { return 4 * (1 + prefill_max_tiles(
 // Tiles of at most 64 rows where they give the two launches at most about two
 // workgroups per CU on average and little more work than the tall ones: the
 // launches then last about as long as their longest tile.  Beyond that the tall
-// tile's fewer code expansions per row win, at 8 bits sooner.  The bucketing
-// counts the tiles, so uneven loads count as they are.  Measured (SwitchGLU, us,
-// tall | half; even loads, then all rows in an eighth of the experts): 1024 x
-// 1024, E 32, k 4, 4 bits: T = 614 56 | 50, 64 | 49, T = 1024 70 | 72, 68 | 53, 6
-// bits T = 900 92 | 85, 90 | 66; 2048 x 2048, E 8, k 2: T = 512 103 | 68, T = 1126
-// 108 | 110 (uneven 118 | 110); 4096 x 1024, E 8, k 2, T = 1126 129 | 117; 2048 x
-// 768, E 128, k 8, T = 280 (mostly one tile a bucket: the same) 115 | 115, 84 |
-// 60.  Past the limits: 1024 x 512, E 64, k 6, T = 1300 64 | 78, 8 bits 67 | 94;
-// 8 bits, 1024 x 1024, T = 1024 73 | 82; 2048 x 512, E 512, k 10, T = 900, an
-// eighth busy 111 | 129.
+// tile's fewer code expansions per row win, sooner at 8 bits, and where K is short
+// and a tile's prologue and epilogue weigh more.  The bucketing counts the tiles,
+// so uneven loads count as they are.  Measured (SwitchGLU of K x N, us, tall |
+// half, 4 bits, even loads unless noted):
+//   1024 x 1024, E 32, k 4: T = 614 56 | 50 (an eighth of the experts busy 64 |
+//     49), T = 1024 70 | 72 (68 | 53); 6 bits T = 900 92 | 85
+//   2048 x 2048, E 8, k 2: T = 512 103 | 68, T = 1126 108 | 110 (uneven 118 | 110),
+//     T = 1250 120 | 111
+//   4096 x 1024, E 8, k 2: T = 1126 129 | 117; 2048 x 256, E 32, k 4: T = 1200 1 | 0.81
+//   2304 x 1536, E 8, k 2: T = 1250 1 | 1.05 (an eighth busy 1 | 0.88)
+//   at the limit: 2048 x 1024, E 16, k 4, T = 900 1 | 0.90, uneven 1 | 1.06; 4096 x
+//     2048, E 8, k 2, T = 900 1 | 0.89, uneven 1 | 1.09
+//   2048 x 768, E 128, k 8: T = 280 115 | 115 (mostly one tile a bucket; 84 | 60)
+// Past the limits:
+//   1024 x 512, E 64, k 6: T = 1300 64 | 78, 8 bits 67 | 94; 1024 x 1024, 8 bits, T =
+//     1024 73 | 82; 2048 x 1024, E 16, k 4: T = 1000 1 | 1.12; 2048 x 512, E 512, k
+//     10, T = 900, an eighth busy: 111 | 129
 HalfTiles prefill_half_max(int64_t P, int E, const moe_qweight* gate, const moe_qweight* down) {
   const int nt = gate->N / (kBN / 2) + down->N / kBN;  // workgroups of a tile
-  return {static_cast<int>(std::min<int64_t>(1040 / nt, prefill_max_tiles(P, E))),
-          2 * (gate->bits == 8 ? 720 : 900) / nt};
+  const bool deep = gate->K >= 2048;
+  const int wgs = deep ? 1160 : 1040;  // (64-row tiles)
+  // 32-row units, halved
+  const int units = gate->bits == 8 ? (deep ? 780 : 720) : deep ? 1000 : 900;
+  return {static_cast<int>(std::min<int64_t>(wgs / nt, prefill_max_tiles(P, E))), 2 * units / nt};
 }
 
 bool prefill_supported(const moe_qweight* w0, const moe_qweight* w1) {
