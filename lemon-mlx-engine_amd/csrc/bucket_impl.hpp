@@ -163,25 +163,16 @@ __device__ void finish_offsets(const int* tot, int64_t P, int E, int* offs_lds, 
     if (e < E && e >= na) rec[e] = make_int4(0, 0, 0, 0);
     if (e == 0 && o.num_active) o.num_active[0] = na;
   }
-  if (o.tiles) {  // the large-bucket GEMM's token-tile table
-    int n4 = n.y, n3 = n.w & 0xffff, n2 = n.w >> 16, n1 = n.z >> 16;
-    int b4 = ex.y, b3 = ex.w & 0xffff, b2 = ex.w >> 16, b1 = ex.z >> 16;
-    // tiles of at most 64 rows: a 128-row one as two, a 96-row one as 64 + 32 (so
-    // their prefixes follow from the scan)
-    const bool half = o.half_max.tiles > 0 && 2 * (n4 + n3) + n2 + n1 <= o.half_max.tiles &&
+  if (__builtin_expect(o.tiles != nullptr, 0)) {  // the large-bucket GEMM's token-tile table (out of line)
+    const int n4 = n.y, n3 = n.w & 0xffff, n2 = n.w >> 16, n1 = n.z >> 16;
+    // tiles of at most 64 rows: a 128-row one as two, a 96-row one as 64 + 32
+    const bool half = 2 * (n4 + n3) + n2 + n1 <= o.half_max.tiles &&
                       4 * n4 + 3 * n3 + 2 * n2 + n1 <= o.half_max.units;  // (uniform)
-    if (half) {
-      c1 += c3;
-      b1 += b3;
-      n1 += n3;
-      c2 += 2 * c4 + c3;
-      b2 += 2 * b4 + b3;
-      n2 += 2 * n4 + n3;
-      c4 = b4 = n4 = c3 = b3 = n3 = 0;
-    }
-    if (e == 0) reinterpret_cast<int4*>(o.tiles)[0] = make_int4(n4, n3, n2, n1);
+    if (e == 0)
+      reinterpret_cast<int4*>(o.tiles)[0] = half ? make_int4(0, 0, 2 * n4 + n3 + n2, n3 + n1) : make_int4(n4, n3, n2, n1);
     if (e <= E)
-      write_tiles(o.tiles, e < E ? e : -1, e < E ? ex.x : 0, ct, half, c4, c3, c2, c1, b4, b3, b2, b1, n4, n3, n2);
+      write_tiles(o.tiles, e < E ? e : -1, e < E ? ex.x : 0, ct, half, c4, c3, c2, c1, ex.y, ex.w & 0xffff,
+                  ex.w >> 16, ex.z >> 16, n4, n3, n2);
   }
   __syncthreads();
 }

@@ -27,14 +27,16 @@ __device__ __forceinline__ void tile_counts(int c, int& c4, int& c3, int& c2, in
   c1 = units == 1 ? 1 : 0;
 }
 // Expert e's entries (bucket at sorted row o0, c rows); b4/b3/b2/b1 = its
-// first index within each class, n4/n3/n2 = the class totals.  half: tiles of at
-// most 64 rows (HalfTiles; no c4, c3).
+// first index within each class, n4/n3/n2 = the class totals.  half: the same in
+// tiles of at most 64 rows (HalfTiles), a 128-row one as two, a 96-row one as 64 +
+// 32 rows, so that their indices follow from these.
 __device__ __forceinline__ void write_tiles(int32_t* tiles, int e, int o0, int c, bool half, int c4, int c3, int c2,
                                             int c1, int b4, int b3, int b2, int b1, int n4, int n3, int n2) {
   int4* tab = reinterpret_cast<int4*>(tiles) + 1;
   if (half) {
-    for (int j = 0; j < c2; ++j) tab[b2 + j] = make_int4(e, o0 + 64 * j, min(64, c - 64 * j), 0);
-    if (c1) tab[n2 + b1] = make_int4(e, o0 + 64 * c2, c - 64 * c2, 0);
+    const int h2 = 2 * c4 + c3 + c2, first = 2 * b4 + b3 + b2;
+    for (int j = 0; j < h2; ++j) tab[first + j] = make_int4(e, o0 + 64 * j, min(64, c - 64 * j), 0);
+    if (c3 + c1) tab[2 * n4 + n3 + n2 + b3 + b1] = make_int4(e, o0 + 64 * h2, c - 64 * h2, 0);
     return;
   }
   for (int j = 0; j < c4; ++j) tab[b4 + j] = make_int4(e, o0 + 128 * j, min(128, c - 128 * j), 0);
